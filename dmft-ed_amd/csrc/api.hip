@@ -670,13 +670,13 @@ extern "C" int dmed_gf_add_chain(double peso_bz, double ei, const double *alpha,
                                  double *greal)
 {
     if (nlanc <= 0) return 0;
-    std::vector<double> d(alpha, alpha + nlanc), e(nlanc, 0.0), z(nlanc);
-    for (int i = 1; i < nlanc; ++i) e[i] = beta[i];
-    if (tql2_first_row(nlanc, d.data(), e.data(), z.data()))
-        return fail(DMED_ENOCONV, "tql2 did not converge");
-    for (auto &x : z) x = x * x;
-    gf_add_poles(peso_bz, ei, d.data(), z.data(), nlanc, isign, wm, lmats, wr, lreal, eps, gmats,
-                 greal);
+    const int lm = std::max(lmats, 0), lr = std::max(lreal, 0);
+    std::vector<double> g(2 * ((size_t)lm + lr));
+    if (int rc = gf_sum({GfTerm{alpha, beta, nlanc, isign, ei, peso_bz, 0.0}}, wm, lm, wr, lr, eps,
+                        g.data()))
+        return rc;
+    for (size_t i = 0; i < 2 * (size_t)lm; ++i) gmats[i] += g[i];
+    for (size_t i = 0; i < 2 * (size_t)lr; ++i) greal[i] += g[2 * (size_t)lm + i];
     return 0;
 }
 

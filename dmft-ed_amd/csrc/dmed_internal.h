@@ -124,6 +124,7 @@ constexpr int kSlotDeflX = 7;           // eigenvectors collected over rounds
 constexpr int kSlotOpTable = 8;         // c / c^+ source-target tables
 constexpr int kSlotStart = 9;           // GF chain start vector
 constexpr int kSlotMid = 10;            // intermediate vector of a two-operator start vector
+constexpr int kSlotGf = 11;             // coefficients, frequencies and results of a G sum
 constexpr int kSlotChainLo = 12;        // 12..14: FP32 tail of a mixed chain
 constexpr int kExecSlots = 16;
 constexpr int kMixedHead = 32;          // FP64 steps at the head of a mixed chain
@@ -300,6 +301,17 @@ int tql2_first_row(int n, double *d, double *e, double *z1);
 void gf_add_poles(double peso, double ei, const double *lam, const double *w2, int n,
                   int isign, const double *wm, int lmats, const double *wr, int lreal,
                   double eps, double *gm, double *gr);
+// One chain of a Green's function: weight pr + i pi on
+// <e1| (z - isign*(T - ei))^-1 |e1>, T of alpha[0..n), beta[1..n).
+struct GfTerm {
+    const double *alpha, *beta;
+    int n, isign;
+    double ei, pr, pi;
+};
+// sum of the terms on both axes (gf.hip): g[0..lm) at i*wm, g[lm..lm+lr) at
+// wr + i*eps, interleaved complex, overwritten
+int gf_sum(const std::vector<GfTerm> &terms, const double *wm, int lm, const double *wr, int lr,
+           double eps, double *g);
 // one branch of the susceptibility pole sums (build_chi_spin.f90:186-250,
 // build_chi_dens.f90:505-733): complex weight pr + i pi, iv = 0 term signed
 // by iv0_sign; vm[0..nv), tau[0..ntau), wr[0..lreal); chi_iv, chi_w

@@ -208,25 +208,6 @@ int run_tasks(int batched, int ntask, const std::function<void(int)> &fn)
     return 0;
 }
 
-// Host-only parallel loop (no device context): tasks write disjoint outputs,
-// so the result does not depend on the thread count.
-void host_parallel(int ntask, const std::function<void(int)> &fn)
-{
-    int nw = (int)std::min<unsigned>(16u, std::max(1u, std::thread::hardware_concurrency()));
-    nw = std::min(nw, ntask);
-    if (nw <= 1) {
-        for (int k = 0; k < ntask; ++k) fn(k);
-        return;
-    }
-    std::atomic<int> next(0);
-    std::vector<std::thread> th;
-    for (int w = 0; w < nw; ++w)
-        th.emplace_back([&]() {
-            for (int k; (k = next.fetch_add(1)) < ntask;) fn(k);
-        });
-    for (auto &t : th) t.join();
-}
-
 double now()
 {
     return std::chrono::duration<double>(std::chrono::steady_clock::now().time_since_epoch()).count();
@@ -577,7 +558,6 @@ extern "C" int dmed_solve(const dmed_solve_params *p, dmed_solve_out *out)
         int nlanc = 0, rc = 0;
         double norm2 = 0.0;
         std::vector<double> al, bl;
-        std::vector<double> lam, w2;    // poles: tql2 eigenvalues and Z(1,j)^2
         std::string err;
     };
     std::vector<Chain> chains;
@@ -689,16 +669,6 @@ extern "C" int dmed_solve(const dmed_solve_params *p, dmed_solve_out *out)
             int nsteps = 0;
             ch.rc = chain_run(ch.J, v.data, DMED_FP64, ch.nlanc, p->prec_gf, 1e-13, ch.al.data(),
                               ch.bl.data(), &nsteps, p->gf_fp64_head);
-            // poles of the chain (add_to_lanczos_gf_normal: tql2 with Z = I)
-            if (!ch.rc) {
-                ch.lam = ch.al;
-                std::vector<double> e(ch.nlanc, 0.0);
-                for (int i = 1; i < ch.nlanc; ++i) e[i] = ch.bl[i];
-                ch.w2.assign(ch.nlanc, 0.0);
-                if (tql2_first_row(ch.nlanc, ch.lam.data(), e.data(), ch.w2.data()))
-                    ch.rc = fail(DMED_ENOCONV, "tql2 did not converge");
-                for (auto &z : ch.w2) z *= z;
-            }
         }
         if (ch.rc) ch.err = dmed_last_error();
     };
@@ -709,35 +679,30 @@ extern "C" int dmed_solve(const dmed_solve_params *p, dmed_solve_out *out)
     // full orbital matrices G[s][a][b] (hybrid bath), interleaved complex
     std::vector<double> gfm(offdiag ? 2 * (size_t)nspin * norb * norb * lm : 0),
         gfr(offdiag ? 2 * (size_t)nspin * norb * norb * lr : 0);
+    std::vector<double> gsum(2 * ((size_t)lm + lr));
+    // a chain's term of G with its Boltzmann weight (kind 2: times -i)
+    auto term_of = [&](const Chain &ch) {
+        const State &st = sl.items[ch.state];
+        double peso = 0.0;
+        if (finite_t) {
+            if (beta * (st.e - egs) < 200) peso = ch.norm2 * std::exp(-beta * (st.e - egs)) / zeta;
+        } else {
+            peso = ch.norm2 / zeta;
+        }
+        return GfTerm{ch.al.data(), ch.bl.data(), ch.nlanc, ch.isign, st.e,
+                      ch.kind == 2 ? 0.0 : peso, ch.kind == 2 ? -peso : 0.0};
+    };
     for (int s = 0; s < nspin && !rc; ++s)
         for (int a = 0; a < norb && !rc; ++a) {
-            std::fill(gm.begin(), gm.end(), 0.0);
-            std::fill(gr.begin(), gr.end(), 0.0);
-            // pole sums of the chains of (s, a), in chain order for every
-            // frequency, split over frequency blocks (deterministic either way)
-            struct Term { const Chain *ch; double peso, e; };
-            std::vector<Term> terms;
+            // the chains of (s, a), in chain order
+            std::vector<GfTerm> terms;
             for (auto &ch : chains) {
                 if (ch.kind != 0 || ch.s != s || ch.a != a || !(ch.norm2 > 0.0)) continue;
-                const State &st = sl.items[ch.state];
-                double peso = 0.0;
-                if (finite_t) {
-                    if (beta * (st.e - egs) < 200) peso = ch.norm2 * std::exp(-beta * (st.e - egs)) / zeta;
-                } else {
-                    peso = ch.norm2 / zeta;
-                }
-                terms.push_back({&ch, peso, st.e});
+                terms.push_back(term_of(ch));
             }
-            const int nfreq = lm + lr, nblk = std::max(1, std::min(64, nfreq / 64));
-            host_parallel(nblk, [&](int b) {
-                const int f0 = (int)((int64_t)nfreq * b / nblk), f1 = (int)((int64_t)nfreq * (b + 1) / nblk);
-                const int m0 = std::min(f0, lm), m1 = std::min(f1, lm);
-                const int r0 = std::max(f0, lm) - lm, r1 = std::max(f1, lm) - lm;
-                for (const Term &t : terms)
-                    gf_add_poles(t.peso, t.e, t.ch->lam.data(), t.ch->w2.data(), t.ch->nlanc,
-                                 t.ch->isign, wm.data() + m0, m1 - m0, wr.data() + r0, r1 - r0,
-                                 p->eps, gm.data() + 2 * m0, gr.data() + 2 * r0);
-            });
+            if ((rc = gf_sum(terms, wm.data(), lm, wr.data(), lr, p->eps, gsum.data()))) break;
+            std::copy(gsum.begin(), gsum.begin() + 2 * (size_t)lm, gm.begin());
+            std::copy(gsum.begin() + 2 * (size_t)lm, gsum.end(), gr.begin());
             for (int l = 0; l < lm && out->gmats; ++l) {
                 const size_t o = gidx(s, s, a, a, l, nspin, norb);
                 out->gmats[2 * o] = gm[2 * l];
@@ -783,33 +748,17 @@ extern "C" int dmed_solve(const dmed_solve_params *p, dmed_solve_out *out)
     // (get_sigma_normal.f90:40-56) with G0^-1 = (z + xmu) 1 - Hloc - Delta,
     // Delta_ab = sum_k V_a(k) V_b(k)/(z - e_k) (ED_BATH_FUNCTIONS.f90:1836-1848, 294-310).
     for (int s = 0; s < nspin && !rc && offdiag; ++s) {
-        for (int a = 0; a < norb; ++a)
-            for (int b = a + 1; b < norb; ++b) {
-                std::vector<double> am(2 * (size_t)lm, 0.0), ar(2 * (size_t)lr, 0.0),
-                    tm(2 * (size_t)lm), tr(2 * (size_t)lr);
+        for (int a = 0; a < norb && !rc; ++a)
+            for (int b = a + 1; b < norb && !rc; ++b) {
+                std::vector<GfTerm> terms;
                 for (auto &ch : chains) {
                     if (ch.kind == 0 || ch.s != s || ch.a != a || ch.b != b || !(ch.norm2 > 0.0))
                         continue;
-                    const State &st = sl.items[ch.state];
-                    double peso = 0.0;
-                    if (finite_t) {
-                        if (beta * (st.e - egs) < 200) peso = ch.norm2 * std::exp(-beta * (st.e - egs)) / zeta;
-                    } else {
-                        peso = ch.norm2 / zeta;
-                    }
-                    if (ch.kind == 1) {
-                        gf_add_poles(peso, st.e, ch.lam.data(), ch.w2.data(), ch.nlanc, ch.isign,
-                                     wm.data(), lm, wr.data(), lr, p->eps, am.data(), ar.data());
-                        continue;
-                    }
-                    // weight -i*peso: (x + i y) += -i (tx + i ty) = ty - i tx
-                    std::fill(tm.begin(), tm.end(), 0.0);
-                    std::fill(tr.begin(), tr.end(), 0.0);
-                    gf_add_poles(peso, st.e, ch.lam.data(), ch.w2.data(), ch.nlanc, ch.isign,
-                                 wm.data(), lm, wr.data(), lr, p->eps, tm.data(), tr.data());
-                    for (int l = 0; l < lm; ++l) { am[2 * l] += tm[2 * l + 1]; am[2 * l + 1] -= tm[2 * l]; }
-                    for (int l = 0; l < lr; ++l) { ar[2 * l] += tr[2 * l + 1]; ar[2 * l + 1] -= tr[2 * l]; }
+                    terms.push_back(term_of(ch));
                 }
+                if ((rc = gf_sum(terms, wm.data(), lm, wr.data(), lr, p->eps, gsum.data()))) break;
+                std::vector<double> am(gsum.begin(), gsum.begin() + 2 * (size_t)lm),
+                    ar(gsum.begin() + 2 * (size_t)lm, gsum.end());
                 auto combine = [&](std::vector<double> &g, const std::vector<double> &full, int L) {
                     const double *ga = full.data() + 2 * (size_t)L * ((s * norb + a) * norb + a);
                     const double *gb = full.data() + 2 * (size_t)L * ((s * norb + b) * norb + b);
@@ -868,7 +817,7 @@ extern "C" int dmed_solve(const dmed_solve_params *p, dmed_solve_out *out)
                     }
             }
         };
-        sigma_axis(gfm, lm, true, out->smats);
+        if (!rc) sigma_axis(gfm, lm, true, out->smats);
         if (!rc) sigma_axis(gfr, lr, false, out->sreal);
     }
     // ---------------------------------------------- spin susceptibility
