@@ -905,13 +905,17 @@ extern "C" int dmed_chi_add_chain(double peso_f, double peso_bz, double ei, cons
     if (!alpha || !beta_l || (nv > 0 && (!vm || !chi_iv)) || (ntau > 0 && (!tau || !chi_tau)) ||
         (lreal > 0 && (!wr || !chi_w)))
         return fail(DMED_EINVAL, "null argument");
-    std::vector<double> d(alpha, alpha + nlanc), e(nlanc, 0.0), z(nlanc);
-    for (int i = 1; i < nlanc; ++i) e[i] = beta_l[i];
-    if (tql2_first_row(nlanc, d.data(), e.data(), z.data()))
-        return fail(DMED_ENOCONV, "tql2 did not converge");
-    for (auto &x : z) x = x * x;
-    chi_add_poles(peso_f, peso_bz, ei, d.data(), z.data(), nlanc, beta, vm, nv, tau, ntau, wr,
-                  lreal, eps, chi_iv, chi_tau, chi_w);
+    const ChiGrid g{vm, tau, wr, std::max(nv, 0), std::max(ntau, 0), std::max(lreal, 0), eps};
+    std::vector<double> o(2 * ((size_t)g.nv + g.nt + g.lr));
+    // S_z is hermitian, so the particle (isign = +1) and hole (-1) terms come
+    // from one chain (build_chi_spin.f90:186-250)
+    std::vector<ChiTerm> terms;
+    for (int isign = 1; isign >= -1; isign -= 2)
+        terms.push_back(ChiTerm{alpha, beta_l, nlanc, 0, isign, 1, peso_f, 0.0, peso_bz, ei});
+    if (int rc = chi_sum(terms, 1, beta, g, o.data())) return rc;
+    for (int i = 0; i < 2 * g.nv; ++i) chi_iv[i] += o[i];
+    for (int i = 0; i < g.nt; ++i) chi_tau[i] += o[2 * ((size_t)g.nv + i)];
+    for (int i = 0; i < 2 * g.lr; ++i) chi_w[i] += o[2 * ((size_t)g.nv + g.nt) + i];
     return 0;
 }
 

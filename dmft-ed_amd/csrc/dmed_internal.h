@@ -312,6 +312,22 @@ struct GfTerm {
 // wr + i*eps, interleaved complex, overwritten
 int gf_sum(const std::vector<GfTerm> &terms, const double *wm, int lm, const double *wr, int lr,
            double eps, double *g);
+// One branch of a susceptibility: the poles of (alpha[0..n), beta[1..n)) with
+// weight (pr + i pi)*peso_bz added to output `target`.
+struct ChiTerm {
+    const double *alpha, *beta;
+    int n, target, isign, iv0_sign;
+    double pr, pi, peso_bz, ei;
+};
+// points of a susceptibility: vm[0..nv), tau[0..nt), wr[0..lr) + i*eps
+struct ChiGrid {
+    const double *vm, *tau, *wr;
+    int nv, nt, lr;
+    double eps;
+};
+// sums of the terms (gf.hip): out[target*(nv+nt+lr) + i], interleaved complex
+// (tau: real part), overwritten
+int chi_sum(std::vector<ChiTerm> terms, int ntarget, double beta, const ChiGrid &g, double *out);
 // one branch of the susceptibility pole sums (build_chi_spin.f90:186-250,
 // build_chi_dens.f90:505-733): complex weight pr + i pi, iv = 0 term signed
 // by iv0_sign; vm[0..nv), tau[0..ntau), wr[0..lreal); chi_iv, chi_w
@@ -320,11 +336,4 @@ void chi_add_branch(double pr, double pi, double peso_bz, double ei, const doubl
                     const double *w2, int n, int isign, int iv0_sign, double beta,
                     const double *vm, int nv, const double *tau, int ntau, const double *wr,
                     int lreal, double eps, double *chi_iv, double *chi_tau, double *chi_w);
-// add_to_lanczos_spinChi (build_chi_spin.f90:186-250) for isign = +1 then -1;
-// vm[0..nv), tau[0..ntau), wr[0..lreal); chi_iv, chi_w interleaved complex
-void chi_add_poles(double peso_f, double peso_bz, double ei, const double *lam, const double *w2,
-                   int n, double beta, const double *vm, int nv, const double *tau, int ntau,
-                   const double *wr, int lreal, double eps, double *chi_iv, double *chi_tau,
-                   double *chi_w);
-
 }  // namespace dmed

@@ -245,17 +245,4 @@ void chi_add_branch(double pr, double pi, double peso_bz, double ei, const doubl
     }
 }
 
-// add_to_lanczos_spinChi (build_chi_spin.f90:186-250).  S_z is hermitian,
-// so the particle (isign = +1) and hole (isign = -1) terms come from one
-// chain, added +1 then -1.
-void chi_add_poles(double peso_f, double peso_bz, double ei, const double *lam, const double *w2,
-                   int n, double beta, const double *vm, int nv, const double *tau, int ntau,
-                   const double *wr, int lreal, double eps, double *chi_iv, double *chi_tau,
-                   double *chi_w)
-{
-    for (int isign = 1; isign >= -1; isign -= 2)
-        chi_add_branch(peso_f, 0.0, peso_bz, ei, lam, w2, n, isign, 1, beta, vm, nv, tau, ntau,
-                       wr, lreal, eps, chi_iv, chi_tau, chi_w);
-}
-
 }  // namespace dmed

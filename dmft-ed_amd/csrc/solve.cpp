@@ -838,6 +838,8 @@ extern "C" int dmed_solve(const dmed_solve_params *p, dmed_solve_out *out)
         for (int i = 0; i < nv; ++i) vm[i] = M_PI / beta * 2.0 * (double)i;
         for (int i = 0; i < nt; ++i) tau[i] = ltau > 0 ? beta * (double)i / (double)ltau : 0.0;
     }
+    const int np = nv + nt + lr;
+    const ChiGrid grid{vm.data(), tau.data(), wr.data(), nv, nt, lr, p->eps};
     for (auto &it : sl.items)
         if ((p->chi_spin || p->chi_dens) && !rc && it.vec->prec != DMED_FP64)
             rc = fail(DMED_ESTATE, "susceptibility start vectors need FP64 states");
@@ -847,7 +849,7 @@ extern "C" int dmed_solve(const dmed_solve_params *p, dmed_solve_out *out)
             int state, row;
             int nlanc = 0, rc = 0;
             double norm2 = 0.0;
-            std::vector<double> lam, w2;
+            std::vector<double> al, bl;
             std::string err;
         };
         std::vector<ChiTask> tasks;
@@ -870,19 +872,11 @@ extern "C" int dmed_solve(const dmed_solve_params *p, dmed_solve_out *out)
             ck.rc = dmed_apply_sz(st.vec, ck.row < norb ? ck.row : -1, &v, &ck.norm2);
             if (!ck.rc && ck.norm2 > 0.0) {
                 ck.nlanc = (int)std::min<int64_t>(S->dim, ngf);
-                std::vector<double> al(ck.nlanc, 0.0), bl(ck.nlanc, 0.0);
+                ck.al.assign(ck.nlanc, 0.0);
+                ck.bl.assign(ck.nlanc, 0.0);
                 int nsteps = 0;
-                ck.rc = chain_run(S, v.data, DMED_FP64, ck.nlanc, p->prec_gf, 1e-13, al.data(),
-                                  bl.data(), &nsteps, p->gf_fp64_head);
-                if (!ck.rc) {
-                    ck.lam = al;
-                    std::vector<double> e(ck.nlanc, 0.0);
-                    for (int i = 1; i < ck.nlanc; ++i) e[i] = bl[i];
-                    ck.w2.assign(ck.nlanc, 0.0);
-                    if (tql2_first_row(ck.nlanc, ck.lam.data(), e.data(), ck.w2.data()))
-                        ck.rc = fail(DMED_ENOCONV, "tql2 did not converge");
-                    for (auto &z : ck.w2) z *= z;
-                }
+                ck.rc = chain_run(S, v.data, DMED_FP64, ck.nlanc, p->prec_gf, 1e-13, ck.al.data(),
+                                  ck.bl.data(), &nsteps, p->gf_fp64_head);
             }
             if (ck.rc) ck.err = dmed_last_error();
         };
@@ -890,29 +884,30 @@ extern "C" int dmed_solve(const dmed_solve_params *p, dmed_solve_out *out)
         for (auto &ck : tasks)
             if (!rc && ck.rc) rc = fail(ck.rc, ck.err);
         if (!rc) {
-            std::vector<double> civ(2 * (size_t)nrow * nv, 0.0), ctau((size_t)nrow * nt, 0.0),
-                cw(2 * (size_t)nrow * lr, 0.0);
+            std::vector<ChiTerm> terms;
             for (auto &ck : tasks) {
                 if (!(ck.norm2 > 0.0)) continue;
                 const State &st = sl.items[ck.state];
-                const double peso_f = ck.norm2 / zeta;
                 const double peso_bz = finite_t ? std::exp(-beta * (st.e - egs)) : 1.0;
-                chi_add_poles(peso_f, peso_bz, st.e, ck.lam.data(), ck.w2.data(), ck.nlanc, beta,
-                              vm.data(), nv, tau.data(), nt, wr.data(), lr, p->eps,
-                              civ.data() + 2 * (size_t)ck.row * nv, ctau.data() + (size_t)ck.row * nt,
-                              cw.data() + 2 * (size_t)ck.row * lr);
+                for (int isign = 1; isign >= -1; isign -= 2)
+                    terms.push_back(ChiTerm{ck.al.data(), ck.bl.data(), ck.nlanc, ck.row, isign, 1,
+                                            ck.norm2 / zeta, 0.0, peso_bz, st.e});
             }
+            std::vector<double> sum(2 * (size_t)nrow * np);
+            rc = chi_sum(terms, nrow, beta, grid, sum.data());
             // Fortran order (Norb+1, L): element (row, i) at row + nrow*i
-            for (int row = 0; row < nrow; ++row) {
+            for (int row = 0; row < nrow && !rc; ++row) {
+                const double *civ = sum.data() + 2 * (size_t)row * np, *ctau = civ + 2 * (size_t)nv,
+                             *cw = ctau + 2 * (size_t)nt;
                 for (int i = 0; i < nv && out->spin_chi_iv; ++i) {
-                    out->spin_chi_iv[2 * ((size_t)row + nrow * i)] = civ[2 * ((size_t)row * nv + i)] / zeta;
-                    out->spin_chi_iv[2 * ((size_t)row + nrow * i) + 1] = civ[2 * ((size_t)row * nv + i) + 1] / zeta;
+                    out->spin_chi_iv[2 * ((size_t)row + nrow * i)] = civ[2 * i] / zeta;
+                    out->spin_chi_iv[2 * ((size_t)row + nrow * i) + 1] = civ[2 * i + 1] / zeta;
                 }
                 for (int i = 0; i < nt && out->spin_chi_tau; ++i)
-                    out->spin_chi_tau[(size_t)row + nrow * i] = ctau[(size_t)row * nt + i] / zeta;
+                    out->spin_chi_tau[(size_t)row + nrow * i] = ctau[2 * i] / zeta;
                 for (int i = 0; i < lr && out->spin_chi_w; ++i) {
-                    out->spin_chi_w[2 * ((size_t)row + nrow * i)] = cw[2 * ((size_t)row * lr + i)] / zeta;
-                    out->spin_chi_w[2 * ((size_t)row + nrow * i) + 1] = cw[2 * ((size_t)row * lr + i) + 1] / zeta;
+                    out->spin_chi_w[2 * ((size_t)row + nrow * i)] = cw[2 * i] / zeta;
+                    out->spin_chi_w[2 * ((size_t)row + nrow * i) + 1] = cw[2 * i + 1] / zeta;
                 }
             }
             out->ltau_used = ltau;
@@ -953,7 +948,7 @@ extern "C" int dmed_solve(const dmed_solve_params *p, dmed_solve_out *out)
             dmed_sector *M = nullptr;       // mix: sector after c_{.,s}
             int nlanc = 0, rc = 0;
             double norm2 = 0.0;
-            std::vector<double> lam, w2;
+            std::vector<double> al, bl;
             std::string err;
         };
         std::vector<DTask> dt;
@@ -1045,19 +1040,11 @@ extern "C" int dmed_solve(const dmed_solve_params *p, dmed_solve_out *out)
             }
             if (!dk.rc && dk.norm2 > 0.0) {
                 dk.nlanc = (int)std::min<int64_t>(dk.kind == kStacked ? I->dim : dk.S->dim, ngf);
-                std::vector<double> al(dk.nlanc, 0.0), bl(dk.nlanc, 0.0);
+                dk.al.assign(dk.nlanc, 0.0);
+                dk.bl.assign(dk.nlanc, 0.0);
                 int nsteps = 0;
-                dk.rc = chain_run(dk.S, buf, DMED_FP64, dk.nlanc, p->prec_gf, 1e-13, al.data(),
-                                  bl.data(), &nsteps, p->gf_fp64_head);
-                if (!dk.rc) {
-                    dk.lam = al;
-                    std::vector<double> e(dk.nlanc, 0.0);
-                    for (int i = 1; i < dk.nlanc; ++i) e[i] = bl[i];
-                    dk.w2.assign(dk.nlanc, 0.0);
-                    if (tql2_first_row(dk.nlanc, dk.lam.data(), e.data(), dk.w2.data()))
-                        dk.rc = fail(DMED_ENOCONV, "tql2 did not converge");
-                    for (auto &z : dk.w2) z *= z;
-                }
+                dk.rc = chain_run(dk.S, buf, DMED_FP64, dk.nlanc, p->prec_gf, 1e-13, dk.al.data(),
+                                  dk.bl.data(), &nsteps, p->gf_fp64_head);
             }
             if (dk.rc) dk.err = dmed_last_error();
         };
@@ -1067,13 +1054,8 @@ extern "C" int dmed_solve(const dmed_solve_params *p, dmed_solve_out *out)
         for (auto &kv : stacked) dmed_sector_free(kv.second);
         if (!rc) {
             const size_t nab = (size_t)norb * norb;
-            // [target][a*norb+b][freq]; tot uses slot 0
-            std::vector<double> civ[3], ctau[3], cw[3];
-            for (int q = 0; q < 3; ++q) {
-                civ[q].assign(2 * nab * nv, 0.0);
-                ctau[q].assign(nab * nt, 0.0);
-                cw[q].assign(2 * nab * lr, 0.0);
-            }
+            // targets [array][a*norb+b]; tot uses slot 0
+            std::vector<ChiTerm> terms;
             for (auto &dk : dt) {
                 if (!(dk.norm2 > 0.0)) continue;
                 const State &st = sl.items[dk.state];
@@ -1083,21 +1065,24 @@ extern "C" int dmed_solve(const dmed_solve_params *p, dmed_solve_out *out)
                 const size_t ab = dk.target == kTot ? 0
                                   : dk.kind == kMix && dk.isign < 0 ? (size_t)dk.b * norb + dk.a
                                                                    : (size_t)dk.a * norb + dk.b;
-                const int q = dk.target;
                 for (int isign = 1; isign >= -1; isign -= 2) {
                     if (dk.isign != 0 && isign != dk.isign) continue;
-                    chi_add_branch(dk.imag ? 0.0 : pf, dk.imag ? pf : 0.0, pbz, st.e, dk.lam.data(),
-                                   dk.w2.data(), dk.nlanc, isign, -isign, beta, vm.data(), nv,
-                                   tau.data(), nt, wr.data(), lr, p->eps, civ[q].data() + 2 * ab * nv,
-                                   ctau[q].data() + ab * nt, cw[q].data() + 2 * ab * lr);
+                    terms.push_back(ChiTerm{dk.al.data(), dk.bl.data(), dk.nlanc,
+                                            (int)(dk.target * nab + ab), isign, -isign,
+                                            dk.imag ? 0.0 : pf, dk.imag ? pf : 0.0, pbz, st.e});
                 }
             }
+            std::vector<double> sum(2 * 3 * nab * np);
+            rc = chi_sum(terms, (int)(3 * nab), beta, grid, sum.data());
+            auto civ = [&](int q, size_t ab) { return sum.data() + 2 * (q * nab + ab) * np; };
+            auto ctau = [&](int q, size_t ab) { return civ(q, ab) + 2 * (size_t)nv; };
+            auto cw = [&](int q, size_t ab) { return civ(q, ab) + 2 * (size_t)(nv + nt); };
             // w(a,b) = 0.5*(w(a,b) - (1+i) w(a,a) - (1+i) w(b,b)), a < b
             for (int a = 0; a < norb; ++a)
                 for (int b = a + 1; b < norb; ++b) {
-                    double *wab = cw[kDens].data() + 2 * ((size_t)a * norb + b) * lr;
-                    const double *waa = cw[kDens].data() + 2 * ((size_t)a * norb + a) * lr;
-                    const double *wbb = cw[kDens].data() + 2 * ((size_t)b * norb + b) * lr;
+                    double *wab = cw(kDens, (size_t)a * norb + b);
+                    const double *waa = cw(kDens, (size_t)a * norb + a);
+                    const double *wbb = cw(kDens, (size_t)b * norb + b);
                     for (int i = 0; i < lr; ++i) {
                         const double xr = waa[2 * i] + wbb[2 * i], xi = waa[2 * i + 1] + wbb[2 * i + 1];
                         const double re = wab[2 * i] - (xr - xi), im = wab[2 * i + 1] - (xr + xi);
@@ -1109,7 +1094,7 @@ extern "C" int dmed_solve(const dmed_solve_params *p, dmed_solve_out *out)
             double *oiv[3] = {out->dens_chi_iv, out->dens_chi_mix_iv, out->dens_chi_tot_iv};
             double *otau[3] = {out->dens_chi_tau, out->dens_chi_mix_tau, out->dens_chi_tot_tau};
             double *ow[3] = {out->dens_chi_w, out->dens_chi_mix_w, out->dens_chi_tot_w};
-            for (int q = 0; q < 3; ++q) {
+            for (int q = 0; q < 3 && !rc; ++q) {
                 const double sc = q == kDens ? zeta : 1.0;
                 const int na = q == kTot ? 1 : norb;
                 for (int a = 0; a < na; ++a)
@@ -1117,14 +1102,14 @@ extern "C" int dmed_solve(const dmed_solve_params *p, dmed_solve_out *out)
                         const size_t ab = (size_t)a * norb + b;
                         const size_t fo = (size_t)a + (size_t)na * b, fs = (size_t)na * na;
                         for (int i = 0; i < nv && oiv[q]; ++i) {
-                            oiv[q][2 * (fo + fs * i)] = civ[q][2 * (ab * nv + i)] / sc;
-                            oiv[q][2 * (fo + fs * i) + 1] = civ[q][2 * (ab * nv + i) + 1] / sc;
+                            oiv[q][2 * (fo + fs * i)] = civ(q, ab)[2 * i] / sc;
+                            oiv[q][2 * (fo + fs * i) + 1] = civ(q, ab)[2 * i + 1] / sc;
                         }
                         for (int i = 0; i < nt && otau[q]; ++i)
-                            otau[q][fo + fs * i] = ctau[q][ab * nt + i] / sc;
+                            otau[q][fo + fs * i] = ctau(q, ab)[2 * i] / sc;
                         for (int i = 0; i < lr && ow[q]; ++i) {
-                            ow[q][2 * (fo + fs * i)] = cw[q][2 * (ab * lr + i)] / sc;
-                            ow[q][2 * (fo + fs * i) + 1] = cw[q][2 * (ab * lr + i) + 1] / sc;
+                            ow[q][2 * (fo + fs * i)] = cw(q, ab)[2 * i] / sc;
+                            ow[q][2 * (fo + fs * i) + 1] = cw(q, ab)[2 * i + 1] / sc;
                         }
                     }
             }

@@ -70,3 +70,41 @@ def test_many_states_solve_vs_oracle():
     assert r["nstates"] == len(o["states"])
     assert np.abs(r["gmats"][0, 0, 0, 0] - o["gmats"][0, 0]).max() < 1e-10
     assert np.abs(r["smats"][0, 0, 0, 0] - o["smats"][0, 0]).max() < 1e-8
+
+
+@pytest.mark.parametrize("n,nv,nt,lr,beta", [(15, 65, 64, 3, 20.0), (16, 1, 1, 1, 20.0), (17, 64, 0, 65, 5.0),
+                                             (200, 0, 1001, 0, 50.0), (301, 1025, 129, 500, 50.0), (1360, 7, 5, 3, 10.0)])
+def test_chi_add_chain_vs_poles(n, nv, nt, lr, beta):
+    print(f"[chi_sum] n={n} nv={nv} nt={nt} lr={lr} beta={beta}", flush=True)
+    rng = np.random.default_rng(n + nv)
+    a = rng.uniform(-0.5, 0.5, n)
+    b = np.concatenate([[0.0], rng.uniform(0.3, 1.2, n - 1)])
+    if n == 200:                                   # a chain that ended at step 150
+        a[150:] = 0.0
+        b[150:] = 0.0
+    ei = -2.0 * np.abs(b).max() - 1.0              # below the chain's levels
+    vm = 2 * np.pi / beta * np.arange(nv)
+    tau = np.linspace(0.0, beta, nt)
+    wr, eps = np.linspace(-4.0, 4.0, lr), 0.1
+    start = rng.standard_normal(nv) + 0j, rng.standard_normal(nt), rng.standard_normal(lr) + 0j
+    iv, ct, cw = (x.copy() for x in start)
+    dmed.chi_add_chain(0.7, 0.9, ei, a, b, beta, vm, tau, wr, eps, iv, ct, cw)
+    lam, w2 = poles(a, b)
+    de, w = lam - ei, 0.63 * w2
+    num = np.exp(-beta * de) - 1.0
+    f = np.where(beta * de < 0.1, beta, -num / de)
+
+    def both(z):
+        return (w * num / (z[:, None] - de) - w * num / (z[:, None] + de)).sum(1)
+
+    want = [start[0] + (both(1j * vm) if nv else 0), start[1] + 0.0, start[2] + (both(wr + 1j * eps) if lr else 0)]
+    if nv:
+        want[0][0] = start[0][0] + 2 * (w * f).sum()
+    if nt:
+        want[1] = start[1] + (w * (np.exp(-tau[:, None] * de) + np.exp(-(beta - tau)[:, None] * de))).sum(1)
+    # errors of the levels of a few units of rounding of ||T||, amplified by
+    # beta in the exponentials and by the squared distance to the poles
+    u = 60 * U * (np.abs(lam).max() + abs(ei))
+    assert (np.abs(iv - want[0]) <= 0.63 * u * 4 / de.min() ** 2 + 16 * U * np.abs(want[0])).all() if nv else True
+    assert (np.abs(ct - want[1]) <= 0.63 * u * 2 * beta + 16 * U * (1 + np.abs(want[1]))).all() if nt else True
+    assert (np.abs(cw - want[2]) <= 0.63 * u * 4 / eps ** 2 + 16 * U * np.abs(want[2])).all() if lr else True
