@@ -464,7 +464,7 @@ static bool use_col_kernel(const dmed_sector *s, int prec)
 // launch or occupancy query, under a lock.  Every launch site calls this
 // first, so concurrent launches from several host threads never see the
 // attribute change under them.
-static int lds_attr_once(const void *kern)
+int lds_attr_once(const void *kern)
 {
     static std::mutex mu;
     static std::map<const void *, hipError_t> done;
