@@ -126,6 +126,7 @@ constexpr int kSlotStart = 9;           // GF chain start vector
 constexpr int kSlotMid = 10;            // intermediate vector of a two-operator start vector
 constexpr int kSlotGf = 11;             // coefficients, frequencies and results of a G sum
 constexpr int kSlotChainLo = 12;        // 12..14: FP32 tail of a mixed chain
+constexpr int kSlotDense = 15;          // matrices of a dense batch
 constexpr int kExecSlots = 16;
 constexpr int kMixedHead = 32;          // FP64 steps at the head of a mixed chain
 
@@ -295,6 +296,32 @@ bool queue_takes(const dmed_sector *s, int neig, int ncv);
 // the queue's buffers (also after a failed launch)
 int queue_launch(SectorQueue &q, hipStream_t st);
 int queue_finish(SectorQueue &q);
+
+// ------------------------------------------------ dense sectors (dense.hip)
+// Sectors diagonalised in full, one workgroup each, in one launch.  The
+// sectors must outlive dense_finish, which waits and fills the items.
+constexpr int64_t kDenseMaxDim = 1024;
+struct DenseItem {
+    const dmed_sector *s = nullptr;
+    int neig = 1;
+    bool lowest = false;                    // lowest level and its copies only
+    double degen = 0.0;
+    bool want_vecs = true;
+    std::vector<double> evals;              // out: ascending
+    std::vector<dmed_vec *> vecs;           // out: nout vectors
+    int nout = 0, rc = 0;                   // out: rc 0 or DMED_ENOCONV
+    const double *dvecs = nullptr;
+};
+struct DenseBatch {
+    std::vector<DenseItem> items;
+    std::vector<unsigned char> tasks;
+    Exec *exec = nullptr;
+    double *dres = nullptr;                 // set once launched
+    size_t nev = 0;
+};
+bool dense_takes(int64_t n);
+int dense_launch(DenseBatch &b, Exec &e);
+int dense_finish(DenseBatch &b);
 
 // ------------------------------------------------------------ host LA
 // symmetric eigen-decomposition of a dense n x n matrix (column-major, in

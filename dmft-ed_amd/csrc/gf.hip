@@ -27,6 +27,7 @@
 #include <vector>
 
 #include "dmed_internal.h"
+#include "tridiag_device.h"
 
 namespace dmed {
 
@@ -185,20 +186,9 @@ struct PoleChain {
     int32_t n, off;
 };
 
-// 1/sqrt(x) for normal x well inside the range: the hardware estimate and
-// three Newton steps y += y/2 (1 - x y^2), each squaring its relative error
-__device__ __forceinline__ double rsqrt_newton(double x)
-{
-    double y = __builtin_amdgcn_rsq(x);
-#pragma unroll
-    for (int k = 0; k < 3; ++k) y = fma(0.5 * y, fma(-x * y, y, 1.0), y);
-    return y;
-}
-
 // Eigenvalues (not sorted) and squared first eigenvector components of the
-// chains' tridiagonal matrices; AB holds (a_k, b_k), b_0 unused.  The 64
-// lanes of a block run the scalar recurrence together (the same values in
-// every lane) and share the scans and shifts.  status: 0, or 1 if an
+// chains' tridiagonal matrices, one wave per block; AB holds (a_k, b_k), b_0
+// unused.  status: 0, or 1 if an
 // eigenvalue took more than 30 iterations.
 __global__ void __launch_bounds__(64) k_chain_poles(const PoleChain *__restrict__ ch,
                                                     const double2 *__restrict__ AB,
@@ -206,6 +196,7 @@ __global__ void __launch_bounds__(64) k_chain_poles(const PoleChain *__restrict_
                                                     int32_t *__restrict__ status)
 {
     extern __shared__ double smem[];
+    __shared__ double sink[kQlSink];
     const PoleChain c0 = ch[blockIdx.x];
     const int n = c0.n, lane = threadIdx.x;
     double *d = smem, *e = smem + n, *z = smem + 2 * n;
@@ -217,92 +208,30 @@ __global__ void __launch_bounds__(64) k_chain_poles(const PoleChain *__restrict_
     }
     if (lane == 0) e[n - 1] = 0.0;
     __syncthreads();
+    const double sc = ql_scale(d, e, n);
+    for (int i = lane; i < n; i += 64) {
+        d[i] *= sc;
+        e[i] *= sc;
+    }
+    __syncthreads();
     double f = 0.0, tst1 = 0.0;
     bool bad = false;
     for (int l = 0; l < n && !bad; ++l) {
         tst1 = fmax(tst1, fabs(d[l]) + fabs(e[l]));
-        // first m >= l with a negligible e_m (e_{n-1} = 0 always is)
-        int m = n - 1;
-        for (int i0 = l; i0 < n; i0 += 64) {
-            const bool hit = i0 + lane < n && tst1 + fabs(e[i0 + lane]) == tst1;
-            const unsigned long long b = __ballot(hit);
-            if (b) {
-                m = i0 + __ffsll(b) - 1;
-                break;
-            }
-        }
+        const int m = ql_find(e, n, l, tst1);
         for (int iter = 0; m != l; ++iter) {
             if (iter >= 30) {
                 bad = true;
                 break;
             }
-            const double el = e[l], dl = d[l], el1 = e[l + 1];
-            double p = (d[l + 1] - dl) / (2.0 * el);
-            double r = sqrt(p * p + 1.0);
-            const double pr = p + (p >= 0.0 ? r : -r);
-            const double nl = el / pr, dl1 = el * pr;
-            const double sh = dl - nl;
-            __syncthreads();
-            if (lane == 0) {
-                d[l] = nl;
-                d[l + 1] = dl1;
-            }
-            for (int i = l + 2 + lane; i < n; i += 64) d[i] -= sh;
-            __syncthreads();
-            f += sh;
-            p = d[m];
-            double c = 1.0, c2 = 1.0, c3 = 1.0, s = 0.0, s2 = 0.0;
-            double zn = z[m];
-            double ei = e[m - 1], di = d[m - 1], zi = z[m - 1];
-            for (int i = m - 1; i >= l; --i) {
-                // the next rotation's operands are loaded ahead of this one's use
-                const int in = i > l ? i - 1 : l;
-                const double en = e[in], dn = d[in], zp = z[in];
-                c3 = c2;
-                c2 = c;
-                s2 = s;
-                const double g = c * ei, h = c * p;
-                const double h2 = fma(p, p, ei * ei);
-                double inv;
-                if (h2 > 1e-280 && h2 < 1e280) {
-                    inv = rsqrt_newton(h2);
-                    r = h2 * inv;
-                } else {
-                    r = hypot(p, ei);
-                    inv = 1.0 / r;
-                }
-                const double eo = s * r;
-                s = ei * inv;
-                c = p * inv;
-                p = c * di - s * g;
-                const double dout = h + s * (c * g + s * di);
-                const double zo = s * zi + c * zn;
-                zn = c * zi - s * zn;
-                if (lane == 0) {
-                    e[i + 1] = eo;
-                    d[i + 1] = dout;
-                    z[i + 1] = zo;
-                }
-                ei = en;
-                di = dn;
-                zi = zp;
-            }
-            p = -s * s2 * c3 * el1 * e[l] / dl1;
-            const double nel = s * p, ndl = c * p;
-            __syncthreads();
-            if (lane == 0) {
-                e[l] = nel;
-                d[l] = ndl;
-                z[l] = zn;
-            }
-            __syncthreads();
-            if (!(tst1 + fabs(nel) > tst1)) break;
+            const double el = ql_iterate<false>(d, e, n, l, m, f, nullptr, nullptr, z, sink);
+            if (!(tst1 + el > tst1)) break;
         }
-        __syncthreads();
+        wave_lds_fence();
         if (lane == 0) d[l] += f;
-        __syncthreads();
+        wave_lds_fence();
     }
-    for (int i = lane; i < n; i += 64) poles[c0.off + i] = make_double2(d[i], z[i] * z[i]);
+    for (int i = lane; i < n; i += 64) poles[c0.off + i] = make_double2(d[i] / sc, z[i] * z[i]);
     if (lane == 0) status[blockIdx.x] = bad ? 1 : 0;
 }
 

@@ -1524,6 +1524,29 @@ int eigh_sector_ex(const dmed_sector *s, int neig, int ncv, int maxit, double to
     const int64_t n = s->dim;
     if (neig < 1 || neig > n) return fail(DMED_EINVAL, "neig out of range");
     if (n <= dense_threshold || neig == n) {
+        // one sector alone: the device from 150 states on (147 states take
+        // 4.9 ms on the host and 5.1 ms here, 225 take 17.2 and 12.0 ms, 400
+        // take 94 and 40 ms)
+        if (n >= 150 && dense_takes(n)) {
+            DenseBatch b;
+            b.items.resize(1);
+            DenseItem &it = b.items[0];
+            it.s = s;
+            it.neig = neig;
+            it.lowest = lowest_multiplet;
+            it.degen = degen;
+            it.want_vecs = evecs != nullptr;
+            if (dense_launch(b, ex()) == 0 && dense_finish(b) == 0 && it.rc == 0) {
+                *nout = it.nout;
+                for (int q = 0; q < it.nout; ++q) {
+                    evals[q] = it.evals[q];
+                    if (resid) resid[q] = 0.0;
+                    if (evecs) evecs[q] = it.vecs[q];
+                }
+                return 0;
+            }
+            for (dmed_vec *v : it.vecs) dmed_vec_free(v);
+        }
         if (!lowest_multiplet) {
             *nout = neig;
             return dense_eigh(s, neig, evals, evecs, resid);

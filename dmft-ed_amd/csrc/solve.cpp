@@ -119,6 +119,9 @@ inline size_t gidx(int s1, int s2, int a, int b, int l, int nspin, int norb)
 // distinct ones; at most kPoolKeep idle contexts are kept, and the rest are
 // destroyed on release.  exec_pool_clear (dmed_finalize) destroys them all.
 constexpr int kPoolKeep = 16;
+// work space of the dense sectors of one launch; sectors past it are solved
+// one by one
+constexpr size_t kDenseBatchBytes = (size_t)256 << 20;
 std::mutex g_pool_mu;
 std::vector<Exec *> g_pool;
 
@@ -384,8 +387,11 @@ extern "C" int dmed_solve(const dmed_solve_params *p, dmed_solve_out *out)
         // Batched form: the small Krylov sectors go to one launch of the
         // persistent work-queue solver on a stream of their own, while the
         // host workers take the rest (largest first) on theirs.
+        // The dense sectors go to one launch, too, on a third stream.
         SectorQueue q;
-        std::vector<int> qsec, rest;
+        DenseBatch db;
+        std::vector<int> qsec, dsec, rest;
+        size_t dense_bytes = 0;
         const char *q_env = std::getenv("DMED_SECTOR_QUEUE");
         const bool use_queue = p->batched && !(q_env && q_env[0] == '0');
         for (int is : order) {
@@ -393,7 +399,17 @@ extern "C" int dmed_solve(const dmed_solve_params *p, dmed_solve_out *out)
             const int ne = (int)std::min<int64_t>(dim, neigen[is]);
             const int nblock = (int)std::min<int64_t>(dim, p->lanc_ncv_factor * ne + p->lanc_ncv_add);
             const int ncv = std::max(nblock, 2 * ne + 10);
-            if (use_queue && dim > p->lanc_dim_threshold && ne < dim &&
+            if ((dim <= p->lanc_dim_threshold || ne == dim) && dense_takes(dim) &&
+                dense_bytes + 16 * (size_t)dim * dim <= kDenseBatchBytes) {
+                dense_bytes += 16 * (size_t)dim * dim;
+                DenseItem it;
+                it.s = secs[is];
+                it.neig = ne;
+                it.lowest = !finite_t;
+                it.degen = 10.0 * p->gs_threshold;
+                db.items.push_back(std::move(it));
+                dsec.push_back(is);
+            } else if (use_queue && dim > p->lanc_dim_threshold && ne < dim &&
                 queue_takes(secs[is], ne, ncv)) {
                 QueueItem it;
                 it.s = secs[is];
@@ -409,6 +425,12 @@ extern "C" int dmed_solve(const dmed_solve_params *p, dmed_solve_out *out)
                 rest.push_back(is);
             }
         }
+        std::vector<Exec *> dex;
+        int drc = 0;
+        if (!db.items.empty()) {
+            drc = pool_acquire(1, dex);
+            if (!drc) drc = dense_launch(db, *dex[0]);
+        }
         hipStream_t qs = nullptr;
         const double tq0 = now();
         int qrc = 0;
@@ -418,6 +440,24 @@ extern "C" int dmed_solve(const dmed_solve_params *p, dmed_solve_out *out)
             if (!qrc) qrc = queue_launch(q, qs);
         }
         rc = run_tasks(p->batched, (int)rest.size(), [&](int k) { solve_sector(rest[k]); });
+        if (!drc) drc = dense_finish(db);
+        if (!dex.empty()) {
+            hipStreamSynchronize(dex[0]->stream);
+            pool_release(dex);
+        }
+        for (size_t k = 0; k < dsec.size() && !rc; ++k) {
+            DenseItem &it = db.items[k];
+            SectorRes &r = sres[dsec[k]];
+            if (drc || it.rc) {
+                // the batch could not run or did not converge: one by one
+                for (dmed_vec *v : it.vecs) dmed_vec_free(v);
+                solve_sector(dsec[k]);
+                continue;
+            }
+            r.nout = it.nout;
+            r.ev = it.evals;
+            r.vecs = it.vecs;
+        }
         const int frc = queue_finish(q);
         if (!qrc) qrc = frc;
         if (qs) hipStreamDestroy(qs);
