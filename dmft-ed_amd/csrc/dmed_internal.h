@@ -63,8 +63,8 @@ struct SpinTables {
     int32_t *hidx = nullptr;
     double *hval = nullptr;
     float *hval32 = nullptr;
-    // packed form for the persistent column kernel: word = rank<<8 | term<<1 | sign,
-    // with |coefficient| = coef[term]; valid when packed == true
+    // packed form for the persistent column kernel: word = term<<25 | sign<<24 |
+    // rank, with |coefficient| = coef[term]; valid when packed == true
     bool packed = false;
     int ncoef = 0;
     uint32_t *hpk = nullptr;            // [nhop][dim]

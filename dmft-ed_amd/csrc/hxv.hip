@@ -26,6 +26,7 @@
 #include <map>
 #include <mutex>
 #include <tuple>
+#include <type_traits>
 #include <vector>
 
 namespace dmed {
@@ -215,12 +216,22 @@ __global__ void __launch_bounds__(1024) k_hxv(const HxvArgs<T> a)
 // then the diagonal -- the same for every (BS, RPT) and grid, so the launch
 // shape never changes y.  In Lanczos mode each column's <x, y> is reduced on
 // its own and stored at PARTIALS[c]: alpha does not depend on the grid either.
+// Address arithmetic bounds the hop loops as much as the loads do, so a lane's
+// rows are 32-bit offsets against uniform column addresses, and a hop word's
+// upper byte indexes a table of signed coefficients: four VALU operations a
+// hop besides the product, where unpacking and 64-bit addresses took eleven
+// (FP32, D = 1.2e7, two orbitals: 106 -> 81 us; FP64, D = 2.2e6: 26 -> 22 us;
+// the largest sector: FP64 1.98 -> 1.85 ms, FP32 1.06 -> 0.98 ms, back to back).
 // HALVES = 2: steps 2-4 run twice, for the first and the second half of the
 // lane's rows, one neighbour column at a time.  Half the accumulators, loads
 // and hop words are live at once, which brings the kernel within the
 // registers of two workgroups per CU (2*BS/256 waves per SIMD); two
 // workgroups let one's LDS gathers overlap the other's far loads.  The sums
 // are the same, term for term, as with HALVES = 1.
+// LDS ahead of the column: 256 signed coefficients, 8 + 16 doubles
+constexpr int kColScBytes = 256 * 8, kColHeadBytes = kColScBytes + 24 * 8 + 64;
+static_assert(kColHeadBytes % 256 == 0, "the column starts on a DMA boundary");
+
 template <typename T, int MODE, int BS, int RPT, int HALVES = 1>
 __global__ void __launch_bounds__(BS, HALVES == 2 ? 2 * BS / 256 : 1) k_hxv_col(
     const T *__restrict__ X, T *__restrict__ Y, int32_t dup, int32_t ddw, int32_t nhu, int32_t nhd,
@@ -230,11 +241,13 @@ __global__ void __launch_bounds__(BS, HALVES == 2 ? 2 * BS / 256 : 1) k_hxv_col(
     const double *__restrict__ WTAB, int32_t dma16, const ChainScalars *__restrict__ CS,
     double *__restrict__ PARTIALS)
 {
+    // LDS: signed coefficients, the impurity diagonal and reduction buffers at
+    // fixed offsets, then the column
     extern __shared__ __align__(16) unsigned char smem[];
-    T *col = reinterpret_cast<T *>(smem);
-    __shared__ T sc[128];
-    __shared__ double wt[8];
-    __shared__ double red[16];
+    T *sc = reinterpret_cast<T *>(smem);
+    double *wt = reinterpret_cast<double *>(smem + kColScBytes), *red = wt + 8;
+    unsigned char *scol = smem + kColHeadBytes;
+    const T *col = reinterpret_cast<const T *>(scol);
     // neighbour columns in flight: two where the registers allow (FP32 up to
     // 13 rows per lane), else one; FP64 spills at two
     constexpr int HDU = (sizeof(T) == 4 && RPT <= 13) ? 2 : 1;
@@ -243,12 +256,24 @@ __global__ void __launch_bounds__(BS, HALVES == 2 ? 2 * BS / 256 : 1) k_hxv_col(
         if (CS->done) return;
         sx = CS->sx;
     }
-    for (int t = threadIdx.x; t < ncoef; t += blockDim.x) sc[t] = (T)COEF[t];
+    for (int t = threadIdx.x; t < 2 * ncoef; t += blockDim.x)
+        sc[t] = (t & 1) ? -(T)COEF[t >> 1] : (T)COEF[t >> 1];
     const int nper = gridDim.x / 8;                  // workgroups per XCD
     const int xcd = blockIdx.x & 7, loc = blockIdx.x >> 3;
     const int last = dup - 1;
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int colbytes = dup * (int)sizeof(T);
+    // row r of the lane, and an element at a 32-bit byte offset from a uniform
+    // address: one offset register a row and no address arithmetic.  (The
+    // empty asm keeps the offset a 32-bit value inside the loops; widened
+    // ahead of them it would cost a 64-bit add per load.)
+    auto row = [&](int r) { return (uint32_t)min((int)threadIdx.x + r * BS, last); };
+    auto at = [](const auto *base, uint32_t i) {
+        using E = std::remove_cv_t<std::remove_reference_t<decltype(*base)>>;
+        uint32_t byte = i * (uint32_t)sizeof(E);
+        asm("" : "+v"(byte));
+        return *reinterpret_cast<const E *>(reinterpret_cast<const char *>(base) + byte);
+    };
     // impurity bits of the lane's rows, four per register
     constexpr int NP = (RPT + 3) / 4;
     uint32_t imp4[NP];
@@ -279,7 +304,7 @@ __global__ void __launch_bounds__(BS, HALVES == 2 ? 2 * BS / 256 : 1) k_hxv_col(
                 if (off < colbytes)
                     __builtin_amdgcn_global_load_lds(
                         (const __attribute__((address_space(1))) void *)(xc + off),
-                        (__attribute__((address_space(3))) void *)(smem + k * 1024), 16, 0, 0);
+                        (__attribute__((address_space(3))) void *)(scol + k * 1024), 16, 0, 0);
             }
         } else {
             for (int k = wave; k * 256 < colbytes; k += BS / 64) {
@@ -287,7 +312,7 @@ __global__ void __launch_bounds__(BS, HALVES == 2 ? 2 * BS / 256 : 1) k_hxv_col(
                 if (off < colbytes)
                     __builtin_amdgcn_global_load_lds(
                         (const __attribute__((address_space(1))) void *)(xc + off),
-                        (__attribute__((address_space(3))) void *)(smem + k * 256), 4, 0, 0);
+                        (__attribute__((address_space(3))) void *)(scol + k * 256), 4, 0, 0);
             }
         }
         if ((int)threadIdx.x < nimp)
@@ -307,7 +332,7 @@ __global__ void __launch_bounds__(BS, HALVES == 2 ? 2 * BS / 256 : 1) k_hxv_col(
                     T g[RH];
 #pragma unroll
                     for (int r = 0; r < RH; ++r)
-                        g[r] = xj[min((int)threadIdx.x + (rb + r) * BS, last)];
+                        g[r] = at(xj, row(rb + r));
 #pragma unroll
                     for (int r = 0; r < RH; ++r) acc[r] += v * g[r];
                 }
@@ -317,16 +342,13 @@ __global__ void __launch_bounds__(BS, HALVES == 2 ? 2 * BS / 256 : 1) k_hxv_col(
                     __syncthreads();
                 }
                 for (int h = 0; h < nhu; ++h) {
+                    const uint32_t *hw = HU + (int64_t)h * dup;
                     uint32_t w[RH];
 #pragma unroll
                     for (int r = 0; r < RH; ++r)
-                        w[r] = HU[(int64_t)h * dup + min((int)threadIdx.x + (rb + r) * BS, last)];
+                        w[r] = at(hw, row(rb + r));
 #pragma unroll
-                    for (int r = 0; r < RH; ++r) {
-                        T vv = sc[(w[r] >> 1) & 127u];
-                        vv = (w[r] & 1u) ? -vv : vv;
-                        acc[r] += vv * col[w[r] >> 8];
-                    }
+                    for (int r = 0; r < RH; ++r) acc[r] += sc[w[r] >> 24] * col[w[r] & 0xffffffu];
                 }
                 // 4. diagonal and store
 #pragma unroll
@@ -366,7 +388,7 @@ __global__ void __launch_bounds__(BS, HALVES == 2 ? 2 * BS / 256 : 1) k_hxv_col(
 #pragma unroll
                 for (int q = 0; q < HDU; ++q)
 #pragma unroll
-                    for (int r = 0; r < RPT; ++r) g[q][r] = xj[q][min((int)threadIdx.x + r * BS, last)];
+                    for (int r = 0; r < RPT; ++r) g[q][r] = at(xj[q], row(r));
 #pragma unroll
                 for (int r = 0; r < RPT; ++r)
 #pragma unroll
@@ -376,15 +398,12 @@ __global__ void __launch_bounds__(BS, HALVES == 2 ? 2 * BS / 256 : 1) k_hxv_col(
             __builtin_amdgcn_s_waitcnt(0);
             __syncthreads();
             for (int h = 0; h < nhu; ++h) {
+                const uint32_t *hw = HU + (int64_t)h * dup;
                 uint32_t w[RPT];
 #pragma unroll
-                for (int r = 0; r < RPT; ++r) w[r] = HU[(int64_t)h * dup + min((int)threadIdx.x + r * BS, last)];
+                for (int r = 0; r < RPT; ++r) w[r] = at(hw, row(r));
 #pragma unroll
-                for (int r = 0; r < RPT; ++r) {
-                    T vv = sc[(w[r] >> 1) & 127u];
-                    vv = (w[r] & 1u) ? -vv : vv;
-                    acc[r] += vv * col[w[r] >> 8];
-                }
+                for (int r = 0; r < RPT; ++r) acc[r] += sc[w[r] >> 24] * col[w[r] & 0xffffffu];
             }
             // 4. diagonal last, with the lane's own x from LDS
 #pragma unroll
@@ -427,11 +446,11 @@ constexpr int kColMaxRptF64 = 13;
 constexpr int kColMaxRptF32 = 16;
 constexpr int kColMaxRptSmall = 8;
 
-// dynamic LDS of the column kernel: the column rounded up to whole 1 KB DMA
+// dynamic LDS of the column kernel: its head and the column rounded up to whole 1 KB DMA
 // chunks (the last 16-byte-granule chunk may be partial)
 static size_t col_lds_bytes(int64_t dup, size_t esz)
 {
-    return ((size_t)dup * esz + 1023) & ~(size_t)1023;
+    return kColHeadBytes + (((size_t)dup * esz + 1023) & ~(size_t)1023);
 }
 
 static int col_max_rpt(int bs, int prec)
@@ -654,7 +673,10 @@ static TuneChoice tune_get(const dmed_sector *s, int prec)
 // Column-kernel launch shape: lanes, rows per lane, workgroups per CU, grid.
 // Fixed rule: 1024 lanes, as many workgroups per CU as registers and LDS
 // allow, at most two (a third lowered the rate at D_up = 3432), in multiples
-// of the 8 XCDs, never more than the columns.
+// of the 8 XCDs, never more than the columns.  Columns of up to 2048 rows
+// would leave such a lane one or two rows: they take four workgroups of 512
+// lanes, and FP32 ones of up to 1024 rows four of 256 (D_up = 924: FP64 8.7 us
+// with 1024 lanes, 7.8 with 512; FP32 9.5 us, and 6.4 with 256).
 struct ColShape {
     int bs = 1024, rpt = 0, per_cu = 1, fit = 1;
     unsigned grid = 8;
@@ -683,8 +705,9 @@ static ColShape col_shape(const dmed_sector *s, int prec, const TuneChoice &tc)
         c.per_cu = std::max(1, std::min(tc.wgs, f.best()));
         c.tuned = true;
     } else {
-        f = col_fit(s, prec, 1024);
-        c.per_cu = std::max(1, std::min(f.best(), 2));
+        c.bs = s->up.dim > 2048 ? 1024 : (prec == DMED_FP32 && s->up.dim <= 1024) ? 256 : 512;
+        f = col_fit(s, prec, c.bs);
+        c.per_cu = std::max(1, std::min(f.best(), c.bs == 1024 ? 2 : 4));
     }
     c.fit = f.best();
     c.halves = c.per_cu > f.one && f.two >= c.per_cu;

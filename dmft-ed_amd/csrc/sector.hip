@@ -181,8 +181,9 @@ static void spin_terms(const Model &m, int sp, std::vector<HopTerm> &terms,
         }
 }
 
-// Packed hop words from the host tables: target rank (24 bits), index of
-// |coefficient| in t.coef (7 bits), sign; left unpacked (t.packed = false)
+// Packed hop words from the host tables: target rank (low 24 bits), index of
+// |coefficient| in t.coef (7 bits) and sign (top bits, so that the upper byte
+// indexes a table of signed coefficients); left unpacked (t.packed = false)
 // past 2^24 ranks or 128 distinct |coefficients|.
 static int pack_hops(SpinTables &t)
 {
@@ -200,7 +201,7 @@ static int pack_hops(SpinTables &t)
             coef.push_back(a);
             id = (int)coef.size() - 1;
         }
-        pk[q] = ((uint32_t)t.h_hidx[q] << 8) | ((uint32_t)id << 1) | (t.h_hval[q] < 0 ? 1u : 0u);
+        pk[q] = (uint32_t)t.h_hidx[q] | ((uint32_t)id << 25) | (t.h_hval[q] < 0 ? 1u << 24 : 0u);
     }
     if (ok) {
         if (coef.empty()) coef.push_back(0.0);
