@@ -263,19 +263,19 @@ int dmed_sector_dims(const dmed_sector *s, int64_t *dim, int64_t *dim_up, int64_
 {
     if (!s) return fail(DMED_EINVAL, "null sector");
     if (dim) *dim = s->dim;
-    if (dim_up) *dim_up = s->up.dim;
-    if (dim_dw) *dim_dw = s->dw.dim;
+    if (dim_up) *dim_up = s->up->dim;
+    if (dim_dw) *dim_dw = s->dw->dim;
     return 0;
 }
 
 int dmed_sector_map(const dmed_sector *s, int64_t *codes)
 {
     if (!s || !codes) return fail(DMED_EINVAL, "null argument");
-    const int64_t du = s->up.dim, dd = s->dw.dim;
+    const int64_t du = s->up->dim, dd = s->dw->dim;
     for (int64_t id = 0; id < dd; ++id) {
-        const int64_t hi = (int64_t)s->dw.h_str[id] << s->ns;
+        const int64_t hi = (int64_t)s->dw->h_str[id] << s->ns;
         int64_t *o = codes + id * du;
-        for (int64_t iu = 0; iu < du; ++iu) o[iu] = hi | (int64_t)s->up.h_str[iu];
+        for (int64_t iu = 0; iu < du; ++iu) o[iu] = hi | (int64_t)s->up->h_str[iu];
     }
     return 0;
 }
@@ -597,7 +597,7 @@ extern "C" int dmed_apply_op(const dmed_vec *psi, int32_t isite, int32_t dagger,
     hipStream_t st = ex().stream;
     std::vector<int32_t> src;
     std::vector<int8_t> sgn;
-    op_tables(up ? I->up : I->dw, up ? dst->up : dst->dw, p, dagger, src, sgn);
+    op_tables(up ? *I->up : *I->dw, up ? *dst->up : *dst->dw, p, dagger, src, sgn);
     int32_t *dsrc = nullptr;
     if (int rc = exec_buf(ex(), kSlotOpTable, std::max<size_t>(src.size(), 1) * 5, (void **)&dsrc)) return rc;
     int8_t *dsgn = reinterpret_cast<int8_t *>(dsrc + std::max<size_t>(src.size(), 1));
@@ -611,20 +611,20 @@ extern "C" int dmed_apply_op(const dmed_vec *psi, int32_t isite, int32_t dagger,
     if (psi->prec == DMED_FP64) {
         if (up)
             hipLaunchKernelGGL(k_apply_up<double>, dim3(g), dim3(256), 0, st, (const double *)psi->data,
-                               I->up.dim, (double *)out->data, dst->up.dim, dst->dw.dim, dsrc, dsgn,
+                               I->up->dim, (double *)out->data, dst->up->dim, dst->dw->dim, dsrc, dsgn,
                                ex().partials);
         else
             hipLaunchKernelGGL(k_apply_dw<double>, dim3(g), dim3(256), 0, st, (const double *)psi->data,
-                               I->up.dim, (double *)out->data, dst->dw.dim, dsrc, dsgn, gsign,
+                               I->up->dim, (double *)out->data, dst->dw->dim, dsrc, dsgn, gsign,
                                ex().partials);
     } else {
         if (up)
             hipLaunchKernelGGL(k_apply_up<float>, dim3(g), dim3(256), 0, st, (const float *)psi->data,
-                               I->up.dim, (float *)out->data, dst->up.dim, dst->dw.dim, dsrc, dsgn,
+                               I->up->dim, (float *)out->data, dst->up->dim, dst->dw->dim, dsrc, dsgn,
                                ex().partials);
         else
             hipLaunchKernelGGL(k_apply_dw<float>, dim3(g), dim3(256), 0, st, (const float *)psi->data,
-                               I->up.dim, (float *)out->data, dst->dw.dim, dsrc, dsgn, gsign,
+                               I->up->dim, (float *)out->data, dst->dw->dim, dsrc, dsgn, gsign,
                                ex().partials);
     }
     DMED_HIP(hipGetLastError());
@@ -852,11 +852,11 @@ int apply_occ(const dmed_sector *s, int prec, const void *psi, unsigned mask, do
     if (int rc = ensure_partials(4096)) return rc;
     if (prec == DMED_FP64)
         hipLaunchKernelGGL(k_apply_occ<double>, dim3(g), dim3(256), 0, st, (const double *)psi,
-                           s->up.dim, s->dw.dim, s->up.imp, s->dw.imp, mask, wu, wd,
+                           s->up->dim, s->dw->dim, s->up->imp, s->dw->imp, mask, wu, wd,
                            (double *)out, ex().partials);
     else
         hipLaunchKernelGGL(k_apply_occ<float>, dim3(g), dim3(256), 0, st, (const float *)psi,
-                           s->up.dim, s->dw.dim, s->up.imp, s->dw.imp, mask, wu, wd,
+                           s->up->dim, s->dw->dim, s->up->imp, s->dw->imp, mask, wu, wd,
                            (float *)out, ex().partials);
     DMED_HIP(hipGetLastError());
     std::vector<double> h(g);
@@ -931,10 +931,10 @@ extern "C" int dmed_observables(const dmed_vec *psi, double peso, double *dens, 
     if (int rc = ensure_partials(6 * 1024)) return rc;
     if (psi->prec == DMED_FP64)
         hipLaunchKernelGGL(k_obs<double>, dim3(g), dim3(256), 0, st, (const double *)psi->data,
-                           s->up.dim, s->dw.dim, s->up.imp, s->dw.imp, s->norb, ex().partials);
+                           s->up->dim, s->dw->dim, s->up->imp, s->dw->imp, s->norb, ex().partials);
     else
         hipLaunchKernelGGL(k_obs<float>, dim3(g), dim3(256), 0, st, (const float *)psi->data,
-                           s->up.dim, s->dw.dim, s->up.imp, s->dw.imp, s->norb, ex().partials);
+                           s->up->dim, s->dw->dim, s->up->imp, s->dw->imp, s->norb, ex().partials);
     DMED_HIP(hipGetLastError());
     std::vector<double> h((size_t)2 * s->norb * g);
     DMED_HIP(hipMemcpyAsync(h.data(), ex().partials, h.size() * 8, hipMemcpyDeviceToHost, st));
@@ -966,15 +966,15 @@ extern "C" int dmed_local_observables(const dmed_vec *psi, double peso, dmed_loc
     const int no = md.norb, nimp = s->nimp, sd = md.nspin - 1;
     if (nimp > 8) return fail(DMED_EUNSUPP, "local observables: Norb <= 3");
     hipStream_t st = ex().stream;
-    const unsigned g = (unsigned)std::max<int64_t>(1, std::min<int64_t>(1024, s->dw.dim));
+    const unsigned g = (unsigned)std::max<int64_t>(1, std::min<int64_t>(1024, s->dw->dim));
     if (int rc = ensure_partials((size_t)64 * g + 16)) return rc;
     if (psi->prec == DMED_FP64)
         hipLaunchKernelGGL(dmed::k_imp_hist<double>, dim3(g), dim3(256), 0, st,
-                           (const double *)psi->data, s->up.dim, s->dw.dim, s->up.imp, s->dw.imp,
+                           (const double *)psi->data, s->up->dim, s->dw->dim, s->up->imp, s->dw->imp,
                            nimp, ex().partials);
     else
         hipLaunchKernelGGL(dmed::k_imp_hist<float>, dim3(g), dim3(256), 0, st,
-                           (const float *)psi->data, s->up.dim, s->dw.dim, s->up.imp, s->dw.imp,
+                           (const float *)psi->data, s->up->dim, s->dw->dim, s->up->imp, s->dw->imp,
                            nimp, ex().partials);
     DMED_HIP(hipGetLastError());
     std::vector<double> h((size_t)nimp * nimp * g);
@@ -1068,12 +1068,12 @@ extern "C" int dmed_local_observables(const dmed_vec *psi, double peso, dmed_loc
         if (int rc = ensure_partials((size_t)2 * gj + 16)) return rc;
         if (psi->prec == DMED_FP64)
             hipLaunchKernelGGL(dmed::k_jterm_sums<double>, dim3(gj), dim3(256), 0, st,
-                               (const double *)psi->data, s->up.dim, s->dw.dim, s->up.ipair,
-                               s->dw.ipair, no, ex().partials);
+                               (const double *)psi->data, s->up->dim, s->dw->dim, s->up->ipair,
+                               s->dw->ipair, no, ex().partials);
         else
             hipLaunchKernelGGL(dmed::k_jterm_sums<float>, dim3(gj), dim3(256), 0, st,
-                               (const float *)psi->data, s->up.dim, s->dw.dim, s->up.ipair,
-                               s->dw.ipair, no, ex().partials);
+                               (const float *)psi->data, s->up->dim, s->dw->dim, s->up->ipair,
+                               s->dw->ipair, no, ex().partials);
         DMED_HIP(hipGetLastError());
         std::vector<double> hj((size_t)2 * gj);
         DMED_HIP(hipMemcpyAsync(hj.data(), ex().partials, hj.size() * 8, hipMemcpyDeviceToHost, st));

@@ -225,10 +225,10 @@ struct WgShape {
 WgShape wg_shape(const dmed_sector *s, int prec)
 {
     WgShape w;
-    const int64_t dup = s->up.dim, ddw = s->dw.dim;
+    const int64_t dup = s->up->dim, ddw = s->dw->dim;
     if (s->dim < 1 || s->dim > kChainWgMaxDim || dup > 1024) return w;
     const size_t esz = prec == DMED_FP32 ? 4 : 8;
-    w.lds = 3 * 16 * 8 + (size_t)s->dim * esz + ((size_t)s->up.nhop * dup + (size_t)s->dw.nhop * ddw) * (esz + 4);
+    w.lds = 3 * 16 * 8 + (size_t)s->dim * esz + ((size_t)s->up->nhop * dup + (size_t)s->dw->nhop * ddw) * (esz + 4);
     if (w.lds + 1024 > ctx().lds_max) return w;
     for (int bs : {256, 512, 1024}) {
         if (dup > bs) continue;
@@ -250,29 +250,29 @@ int launch_wg(const dmed_sector *s, const WgShape &w, void *vp, void *v, int cou
     WgArgs<T> a;
     a.vp = static_cast<T *>(vp);
     a.v = static_cast<T *>(v);
-    a.dup = (int32_t)s->up.dim;
-    a.ddw = (int32_t)s->dw.dim;
-    a.nhu = s->up.nhop;
-    a.nhd = s->dw.nhop;
+    a.dup = (int32_t)s->up->dim;
+    a.ddw = (int32_t)s->dw->dim;
+    a.nhu = s->up->nhop;
+    a.nhd = s->dw->nhop;
     a.nimp = s->nimp;
     a.groups = w.groups;
     a.count = count;
-    a.hu_idx = s->up.hidx;
-    a.hd_idx = s->dw.hidx;
+    a.hu_idx = s->up->hidx;
+    a.hd_idx = s->dw->hidx;
     if constexpr (sizeof(T) == 8) {
-        a.hu_val = s->up.hval;
-        a.hd_val = s->dw.hval;
+        a.hu_val = s->up->hval;
+        a.hd_val = s->dw->hval;
     } else {
-        a.hu_val = s->up.hval32;
-        a.hd_val = s->dw.hval32;
+        a.hu_val = s->up->hval32;
+        a.hd_val = s->dw->hval32;
     }
-    a.du = s->up.diag;
-    a.dd = s->dw.diag;
+    a.du = s->up->diag;
+    a.dd = s->dw->diag;
     a.W = s->W;
-    a.impu = s->up.imp;
-    a.impd = s->dw.imp;
-    a.ju = s->up.ipair;
-    a.jd = s->dw.ipair;
+    a.impu = s->up->imp;
+    a.impd = s->dw->imp;
+    a.ju = s->up->ipair;
+    a.jd = s->dw->ipair;
     a.norb = s->norb;
     a.jx = s->jx;
     a.jp = s->jp;

@@ -348,21 +348,21 @@ int dense_launch(DenseBatch &b, Exec &e)
         DenseItem &it = b.items[k];
         const dmed_sector *s = it.s;
         DenseTask &t = h[k];
-        t.hu_idx = s->up.hidx;
-        t.hd_idx = s->dw.hidx;
-        t.hu_val = s->up.hval;
-        t.hd_val = s->dw.hval;
-        t.ju = s->up.ipair;
-        t.jd = s->dw.ipair;
-        t.du = s->up.diag;
-        t.dd = s->dw.diag;
+        t.hu_idx = s->up->hidx;
+        t.hd_idx = s->dw->hidx;
+        t.hu_val = s->up->hval;
+        t.hd_val = s->dw->hval;
+        t.ju = s->up->ipair;
+        t.jd = s->dw->ipair;
+        t.du = s->up->diag;
+        t.dd = s->dw->diag;
         t.W = s->W;
-        t.impu = s->up.imp;
-        t.impd = s->dw.imp;
-        t.dup = (int32_t)s->up.dim;
-        t.ddw = (int32_t)s->dw.dim;
-        t.nhu = s->up.nhop;
-        t.nhd = s->dw.nhop;
+        t.impu = s->up->imp;
+        t.impd = s->dw->imp;
+        t.dup = (int32_t)s->up->dim;
+        t.ddw = (int32_t)s->dw->dim;
+        t.nhu = s->up->nhop;
+        t.nhd = s->dw->nhop;
         t.nimp = s->nimp;
         t.jterms = s->jterms;
         t.norb = s->norb;

@@ -5,6 +5,8 @@
 
 #include <cstdint>
 #include <complex>
+#include <map>
+#include <memory>
 #include <string>
 #include <vector>
 
@@ -52,8 +54,14 @@ struct HopTerm {
 
 // Per-spin tables of a sector: strings of n electrons in Ns orbitals in
 // numeric order, their single-spin diagonal energy, impurity bits and hop
-// lists (target rank, signed coefficient) laid out hop-major [h][r].
+// lists (target rank, signed coefficient) laid out hop-major [h][r].  They
+// depend on the spin and its electron count alone, so sectors share them; the
+// last one to go frees the device memory.
 struct SpinTables {
+    SpinTables() = default;
+    SpinTables(const SpinTables &) = delete;
+    SpinTables &operator=(const SpinTables &) = delete;
+    ~SpinTables();
     int n = 0;
     int64_t dim = 0;
     int nhop = 0;
@@ -89,11 +97,12 @@ struct dmed_sector {
     int nup = 0, ndw = 0, ns = 0, norb = 0;
     int64_t dim = 0;
     int model_generation = -1;
-    dmed::SpinTables up, dw;
+    std::shared_ptr<dmed::SpinTables> up, dw;
     int nimp = 1;                       // 2^Norb
     int jterms = 0;                     // spin-exchange / pair-hopping present
     double jx = 0.0, jp = 0.0;
     double *W = nullptr;                // device [nimp*nimp] interaction table W[iu*nimp+id]
+    std::shared_ptr<void> W_own;        // its memory, shared like the spin tables
     std::vector<double> h_W;
 };
 
@@ -168,13 +177,19 @@ int ensure_partials(size_t n);          // on ex()
 int copy_h2d(void *dst, const void *src, size_t bytes);   // on ex().stream, synchronous
 
 // ------------------------------------------------------------- sectors
-int sector_build(dmed_sector *s, int nup, int ndw);
+// Spin tables of one model, built on first use: tables of (spin, electrons)
+// for the sectors of a solve, with spin 0's serving both when Nspin = 1.
+struct SpinCache {
+    std::map<std::pair<int, int>, std::shared_ptr<SpinTables>> m;
+    std::shared_ptr<void> W;                // interaction table
+};
+int sector_build(dmed_sector *s, int nup, int ndw, SpinCache *cache = nullptr);
 // Sector (nup, ndw) stacked twice along the down-spin index: vectors of
 // 2*dim entries [x; y] and H*[x; y] = [H x; H y] (H (+) H).  Built from
 // sector_build with the down-spin tables repeated and their column indices
 // shifted by D_dw in the second copy; for chains of complex start vectors
 // x - i y under the real H, whose Lanczos coefficients are those of [x; y].
-int sector_build_stacked(dmed_sector *s, int nup, int ndw);
+int sector_build_stacked(dmed_sector *s, int nup, int ndw, SpinCache *cache = nullptr);
 // out = (wu*n_up + wd*n_dw)(orbitals in mask) psi on the calling context's
 // stream, norm2 = ||out||^2 (api.hip)
 int apply_occ(const dmed_sector *s, int prec, const void *psi, unsigned mask, double wu,

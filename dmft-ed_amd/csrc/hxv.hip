@@ -462,7 +462,7 @@ static int col_max_rpt(int bs, int prec)
 // rows per lane of a bs-lane column workgroup, 0 when the column does not fit
 static int col_rpt(const dmed_sector *s, int prec, int bs)
 {
-    const int64_t rpt = (s->up.dim + bs - 1) / bs;
+    const int64_t rpt = (s->up->dim + bs - 1) / bs;
     return rpt >= 1 && rpt <= col_max_rpt(bs, prec) ? (int)rpt : 0;
 }
 
@@ -472,10 +472,10 @@ static bool use_col_kernel(const dmed_sector *s, int prec)
 {
     const Context &c = ctx();
     const size_t esz = prec == DMED_FP32 ? 4 : 8;
-    const int64_t dup = s->up.dim;
-    return !s->jterms && s->up.packed && s->up.ncoef <= 128 && s->nimp <= 8 && dup >= 512 &&
+    const int64_t dup = s->up->dim;
+    return !s->jterms && s->up->packed && s->up->ncoef <= 128 && s->nimp <= 8 && dup >= 512 &&
            col_rpt(s, prec, 1024) > 0 && col_lds_bytes(dup, esz) + 2048 <= c.lds_max &&
-           s->dw.dim >= 64;
+           s->dw->dim >= 64;
 }
 
 // A kernel's dynamic-LDS limit is process-wide state: it is raised once per
@@ -580,14 +580,14 @@ static ColFit col_fit(const dmed_sector *s, int prec, int bs)
     // the occupancy query is the same for every sector of this shape: keep it
     static std::mutex mu;
     static std::map<std::tuple<int64_t, int, int>, ColFit> memo;
-    const auto key = std::make_tuple(s->up.dim, prec == DMED_FP32 ? 1 : 0, bs);
+    const auto key = std::make_tuple(s->up->dim, prec == DMED_FP32 ? 1 : 0, bs);
     {
         std::lock_guard<std::mutex> lk(mu);
         auto it = memo.find(key);
         if (it != memo.end()) return it->second;
     }
     const int rpt = col_rpt(s, prec, bs);
-    const size_t shmem = col_lds_bytes(s->up.dim, prec == DMED_FP32 ? 4 : 8);
+    const size_t shmem = col_lds_bytes(s->up->dim, prec == DMED_FP32 ? 4 : 8);
     ColFit f;
     if (rpt == 0) {
         f.one = 0;
@@ -626,7 +626,7 @@ using TuneKey = std::tuple<int64_t, int64_t, int, int, int, int>;
 
 static TuneKey tune_key(const dmed_sector *s, int prec)
 {
-    return TuneKey{s->up.dim, s->dw.dim, s->up.nhop, s->dw.nhop, s->nimp,
+    return TuneKey{s->up->dim, s->dw->dim, s->up->nhop, s->dw->nhop, s->nimp,
                    prec == DMED_FP32 ? DMED_FP32 : DMED_FP64};
 }
 
@@ -688,7 +688,7 @@ static unsigned col_grid_for(const dmed_sector *s, int per_cu)
 {
     const int ncu = std::max(8, ctx().num_cu);
     int g = (ncu / 8) * 8 * per_cu;
-    while (g > 8 && g / 8 > (s->dw.dim + 7) / 8) g -= 8;
+    while (g > 8 && g / 8 > (s->dw->dim + 7) / 8) g -= 8;
     return (unsigned)g;
 }
 
@@ -705,7 +705,7 @@ static ColShape col_shape(const dmed_sector *s, int prec, const TuneChoice &tc)
         c.per_cu = std::max(1, std::min(tc.wgs, f.best()));
         c.tuned = true;
     } else {
-        c.bs = s->up.dim > 2048 ? 1024 : (prec == DMED_FP32 && s->up.dim <= 1024) ? 256 : 512;
+        c.bs = s->up->dim > 2048 ? 1024 : (prec == DMED_FP32 && s->up->dim <= 1024) ? 256 : 512;
         f = col_fit(s, prec, c.bs);
         c.per_cu = std::max(1, std::min(f.best(), c.bs == 1024 ? 2 : 4));
     }
@@ -720,7 +720,7 @@ template <typename T, int MODE>
 static int launch_col(const dmed_sector *s, const void *x, void *y, ChainScalars *cs,
                       double *partials, const ColShape &c, hipStream_t st)
 {
-    const int64_t dup = s->up.dim;
+    const int64_t dup = s->up->dim;
     const size_t shmem = col_lds_bytes(dup, sizeof(T));
     // 16-byte DMA granules need every column start 16-byte aligned
     const int dma16 = ((uintptr_t)x % 16 == 0) && ((size_t)dup * sizeof(T)) % 16 == 0;
@@ -729,10 +729,10 @@ static int launch_col(const dmed_sector *s, const void *x, void *y, ChainScalars
         rc = lds_attr_once((const void *)kern);
         if (rc) return;
         hipLaunchKernelGGL(kern, dim3(c.grid), dim3(c.bs), shmem, st, static_cast<const T *>(x),
-                           static_cast<T *>(y), (int32_t)dup, (int32_t)s->dw.dim,
-                           (int32_t)s->up.nhop, (int32_t)s->dw.nhop, (int32_t)s->nimp,
-                           (int32_t)s->up.ncoef, s->up.hpk, s->up.coef, s->dw.hidx, s->dw.hval,
-                           s->up.diag, s->dw.diag, s->up.imp, s->dw.imp, s->W, (int32_t)dma16,
+                           static_cast<T *>(y), (int32_t)dup, (int32_t)s->dw->dim,
+                           (int32_t)s->up->nhop, (int32_t)s->dw->nhop, (int32_t)s->nimp,
+                           (int32_t)s->up->ncoef, s->up->hpk, s->up->coef, s->dw->hidx, s->dw->hval,
+                           s->up->diag, s->dw->diag, s->up->imp, s->dw->imp, s->W, (int32_t)dma16,
                            (const ChainScalars *)cs, partials);
     });
     if (!ok) return fail(DMED_EINVAL, "column kernel: unsupported rows per lane");
@@ -752,7 +752,7 @@ static LaunchShape pick_shape(const dmed_sector *s, int prec)
 {
     const Context &c = ctx();
     const size_t esz = prec == DMED_FP32 ? 4 : 8;
-    const int64_t dup = s->up.dim, ddw = s->dw.dim;
+    const int64_t dup = s->up->dim, ddw = s->dw->dim;
     LaunchShape sh{};
     const size_t colb = (size_t)dup * esz;
     const size_t wtb = 8 * 64 * (size_t)s->nimp;
@@ -783,29 +783,29 @@ static int launch_t(const dmed_sector *s, const void *x, void *y, ChainScalars *
     HxvArgs<T> a;
     a.x = static_cast<const T *>(x);
     a.y = static_cast<T *>(y);
-    a.dup = (int32_t)s->up.dim;
-    a.ddw = (int32_t)s->dw.dim;
-    a.nhu = s->up.nhop;
-    a.nhd = s->dw.nhop;
+    a.dup = (int32_t)s->up->dim;
+    a.ddw = (int32_t)s->dw->dim;
+    a.nhu = s->up->nhop;
+    a.nhd = s->dw->nhop;
     a.nimp = s->nimp;
     a.cb = sh.cb;
     a.inv_dup = 1.0f / (float)a.dup;
-    a.hu_idx = s->up.hidx;
-    a.hd_idx = s->dw.hidx;
+    a.hu_idx = s->up->hidx;
+    a.hd_idx = s->dw->hidx;
     if constexpr (sizeof(T) == 8) {
-        a.hu_val = reinterpret_cast<const T *>(s->up.hval);
-        a.hd_val = reinterpret_cast<const T *>(s->dw.hval);
+        a.hu_val = reinterpret_cast<const T *>(s->up->hval);
+        a.hd_val = reinterpret_cast<const T *>(s->dw->hval);
     } else {
-        a.hu_val = reinterpret_cast<const T *>(s->up.hval32);
-        a.hd_val = reinterpret_cast<const T *>(s->dw.hval32);
+        a.hu_val = reinterpret_cast<const T *>(s->up->hval32);
+        a.hd_val = reinterpret_cast<const T *>(s->dw->hval32);
     }
-    a.du = s->up.diag;
-    a.dd = s->dw.diag;
-    a.impu = s->up.imp;
-    a.impd = s->dw.imp;
+    a.du = s->up->diag;
+    a.dd = s->dw->diag;
+    a.impu = s->up->imp;
+    a.impd = s->dw->imp;
     a.W = s->W;
-    a.ju = s->up.ipair;
-    a.jd = s->dw.ipair;
+    a.ju = s->up->ipair;
+    a.jd = s->dw->ipair;
     a.jterms = s->jterms;
     a.norb = s->norb;
     a.jx = s->jx;
@@ -925,7 +925,7 @@ void tune_ensure(const dmed_sector *s, int prec, hipStream_t st)
         }
     } else {
         LaunchShape base = pick_shape(s, prec);     // no recorded choice yet: the fixed rule
-        const int64_t dup = s->up.dim, ddw = s->dw.dim;
+        const int64_t dup = s->up->dim, ddw = s->dw->dim;
         const size_t colb = (size_t)dup * esz;
         std::vector<std::pair<int, int>> cand{{base.cb, base.bs}};
         for (int cb = 1; cb <= 64 && cb <= ddw; cb *= 2)
@@ -973,10 +973,10 @@ static LaunchShape tile_shape(const dmed_sector *s, int prec, int mode)
     const TuneChoice tc = tune_get(s, prec);
     if (tc.cb > 0) {
         const size_t esz = prec == DMED_FP32 ? 4 : 8;
-        const int64_t ddw = s->dw.dim;
+        const int64_t ddw = s->dw->dim;
         sh.cb = (int)std::min<int64_t>(tc.cb, std::max<int64_t>(ddw, 1));
         sh.bs = tc.bs;
-        sh.shmem = (sh.lds ? (((size_t)sh.cb * s->up.dim * esz + 15) & ~(size_t)15) : 0) +
+        sh.shmem = (sh.lds ? (((size_t)sh.cb * s->up->dim * esz + 15) & ~(size_t)15) : 0) +
                    8 * (size_t)sh.cb * s->nimp;
         sh.grid = (unsigned)((ddw + sh.cb - 1) / sh.cb);
     }
@@ -992,7 +992,7 @@ int launch_hxv(const dmed_sector *s, const void *x, void *y, int prec, int mode,
     const bool f32 = prec == DMED_FP32;
     if (use_col_kernel(s, prec)) {
         const ColShape c = col_shape(s, prec, tune_get(s, prec));
-        if (nparts) *nparts = (int)s->dw.dim;         // one partial per column
+        if (nparts) *nparts = (int)s->dw->dim;         // one partial per column
         if (f32)
             return mode == kPlain ? launch_col<float, kPlain>(s, x, y, cs, partials, c, st)
                                   : launch_col<float, kLanczos>(s, x, y, cs, partials, c, st);
@@ -1016,7 +1016,7 @@ int launch_hxv(const dmed_sector *s, const void *x, void *y, int prec, int mode,
 // partial sums a Lanczos-mode H*v of s leaves (column kernel: one per column)
 int hxv_nparts(const dmed_sector *s, int prec)
 {
-    if (use_col_kernel(s, prec)) return (int)s->dw.dim;
+    if (use_col_kernel(s, prec)) return (int)s->dw->dim;
     return (int)pick_shape(s, prec).grid;
 }
 
@@ -1040,7 +1040,7 @@ int hxv_shape(const dmed_sector *s, int prec, dmed_hxv_shape *out)
         const LaunchShape sh = tile_shape(s, prec, kPlain);
         out->kernel = 1;
         out->lanes = sh.bs;
-        out->rows_per_lane = (int32_t)((sh.cb * s->up.dim + sh.bs - 1) / sh.bs);
+        out->rows_per_lane = (int32_t)((sh.cb * s->up->dim + sh.bs - 1) / sh.bs);
         out->columns_per_group = sh.cb;
         out->groups_per_cu = 0;
         out->grid = (int32_t)sh.grid;

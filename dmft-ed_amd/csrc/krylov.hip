@@ -1010,20 +1010,20 @@ int tridiag_lowest(int n, const double *a, const double *b, double *theta, doubl
 // diagonalise it
 int dense_eigh(const dmed_sector *s, int neig, double *evals, dmed_vec **evecs, double *resid)
 {
-    const int64_t dup = s->up.dim, ddw = s->dw.dim, n = s->dim;
+    const int64_t dup = s->up->dim, ddw = s->dw->dim, n = s->dim;
     std::vector<double> H((size_t)n * n, 0.0), w(n);
     for (int64_t id = 0; id < ddw; ++id)
         for (int64_t iu = 0; iu < dup; ++iu) {
             const int64_t i = iu + id * dup;
-            H[(size_t)i * n + i] += s->up.h_diag[iu] + s->dw.h_diag[id] +
-                                    s->h_W[s->up.h_imp[iu] * s->nimp + s->dw.h_imp[id]];
-            for (int h = 0; h < s->up.nhop; ++h) {
-                const int64_t j = s->up.h_hidx[(size_t)h * dup + iu] + id * dup;
-                H[(size_t)j * n + i] += s->up.h_hval[(size_t)h * dup + iu];
+            H[(size_t)i * n + i] += s->up->h_diag[iu] + s->dw->h_diag[id] +
+                                    s->h_W[s->up->h_imp[iu] * s->nimp + s->dw->h_imp[id]];
+            for (int h = 0; h < s->up->nhop; ++h) {
+                const int64_t j = s->up->h_hidx[(size_t)h * dup + iu] + id * dup;
+                H[(size_t)j * n + i] += s->up->h_hval[(size_t)h * dup + iu];
             }
-            for (int h = 0; h < s->dw.nhop; ++h) {
-                const int64_t j = iu + (int64_t)s->dw.h_hidx[(size_t)h * ddw + id] * dup;
-                H[(size_t)j * n + i] += s->dw.h_hval[(size_t)h * ddw + id];
+            for (int h = 0; h < s->dw->nhop; ++h) {
+                const int64_t j = iu + (int64_t)s->dw->h_hidx[(size_t)h * ddw + id] * dup;
+                H[(size_t)j * n + i] += s->dw->h_hval[(size_t)h * ddw + id];
             }
             // spin exchange and pair hopping: up pair hop b -> a with down
             // pair hop a -> b (Jx) or b -> a (Jp)
@@ -1032,14 +1032,14 @@ int dense_eigh(const dmed_sector *s, int neig, double *evals, dmed_vec **evecs, 
                 for (int pa = 0; pa < no; ++pa)
                     for (int pb = 0; pb < no; ++pb) {
                         if (pa == pb) continue;
-                        const int32_t wu = s->up.h_ipair[(size_t)(pa * no + pb) * dup + iu];
+                        const int32_t wu = s->up->h_ipair[(size_t)(pa * no + pb) * dup + iu];
                         if (wu < 0) continue;
                         const double su = (wu & 1) ? -1.0 : 1.0;
-                        const int32_t wx = s->dw.h_ipair[(size_t)(pb * no + pa) * ddw + id];
+                        const int32_t wx = s->dw->h_ipair[(size_t)(pb * no + pa) * ddw + id];
                         if (wx >= 0)
                             H[(size_t)((wu >> 1) + (int64_t)(wx >> 1) * dup) * n + i] +=
                                 s->jx * su * ((wx & 1) ? -1.0 : 1.0);
-                        const int32_t wp = s->dw.h_ipair[(size_t)(pa * no + pb) * ddw + id];
+                        const int32_t wp = s->dw->h_ipair[(size_t)(pa * no + pb) * ddw + id];
                         if (wp >= 0)
                             H[(size_t)((wu >> 1) + (int64_t)(wp >> 1) * dup) * n + i] +=
                                 s->jp * su * ((wp & 1) ? -1.0 : 1.0);

@@ -135,6 +135,7 @@ __global__ void k_spin_tables(const uint32_t *__restrict__ str, int64_t dim, int
 
 static void release_spin(SpinTables &t)
 {
+    // device memory only
     hipFree(t.str);
     hipFree(t.diag);
     hipFree(t.imp);
@@ -144,14 +145,15 @@ static void release_spin(SpinTables &t)
     hipFree(t.hpk);
     hipFree(t.coef);
     hipFree(t.ipair);
-    t = SpinTables();
 }
+
+SpinTables::~SpinTables() { release_spin(*this); }
 
 void sector_release(dmed_sector *s)
 {
-    release_spin(s->up);
-    release_spin(s->dw);
-    hipFree(s->W);
+    s->up.reset();
+    s->dw.reset();
+    s->W_own.reset();
     s->W = nullptr;
 }
 
@@ -358,7 +360,24 @@ static int build_pairs(const Model &m, SpinTables &t)
     return 0;
 }
 
-int sector_build(dmed_sector *s, int nup, int ndw)
+// Tables of spin sp with n electrons from the cache, or new ones.  `pairs`:
+// with the impurity pair hops of the spin-exchange terms.
+static int spin_tables(const Model &m, int sp, int n, bool pairs, SpinCache &cache,
+                       std::shared_ptr<SpinTables> &out)
+{
+    auto &e = cache.m[{m.nspin == 2 ? sp : 0, n}];
+    if (!e) {
+        auto t = std::make_shared<SpinTables>();
+        if (int rc = build_spin(m, sp, n, *t, ex().stream)) return rc;
+        if (pairs)
+            if (int rc = build_pairs(m, *t)) return rc;
+        e = std::move(t);
+    }
+    out = e;
+    return 0;
+}
+
+int sector_build(dmed_sector *s, int nup, int ndw, SpinCache *cache)
 {
     Context &c = ctx();
     const Model &m = cur_model();
@@ -370,23 +389,27 @@ int sector_build(dmed_sector *s, int nup, int ndw)
     s->ns = m.ns;
     s->norb = m.norb;
     s->model_generation = m.generation;
-    if (int rc = build_spin(m, 0, nup, s->up, ex().stream)) return rc;
-    if (int rc = build_spin(m, 1, ndw, s->dw, ex().stream)) return rc;
-    s->dim = s->up.dim * s->dw.dim;
-    s->nimp = 1 << m.norb;
     s->jterms = (m.jhflag && m.norb > 1 && (m.jx != 0.0 || m.jp != 0.0)) ? 1 : 0;
+    SpinCache own;
+    SpinCache &sc = cache ? *cache : own;
+    if (int rc = spin_tables(m, 0, nup, s->jterms != 0, sc, s->up)) return rc;
+    if (int rc = spin_tables(m, 1, ndw, s->jterms != 0, sc, s->dw)) return rc;
+    s->dim = s->up->dim * s->dw->dim;
+    s->nimp = 1 << m.norb;
     s->jx = m.jx;
     s->jp = m.jp;
-    if (s->jterms) {
-        if (int rc = build_pairs(m, s->up)) return rc;
-        if (int rc = build_pairs(m, s->dw)) return rc;
-    }
     s->h_W.resize(s->nimp * s->nimp);
     for (int iu = 0; iu < s->nimp; ++iu)
         for (int id = 0; id < s->nimp; ++id)
             s->h_W[iu * s->nimp + id] = interaction(m, iu, id);
-    DMED_HIP(hipMalloc(&s->W, s->h_W.size() * sizeof(double)));
-    if (int rc = copy_h2d(s->W, s->h_W.data(), s->h_W.size() * sizeof(double))) return rc;
+    if (!sc.W) {
+        double *d = nullptr;
+        DMED_HIP(hipMalloc(&d, s->h_W.size() * sizeof(double)));
+        sc.W = std::shared_ptr<void>(d, [](void *p) { hipFree(p); });
+        if (int rc = copy_h2d(d, s->h_W.data(), s->h_W.size() * sizeof(double))) return rc;
+    }
+    s->W_own = sc.W;
+    s->W = static_cast<double *>(s->W_own.get());
     return 0;
 }
 
@@ -463,12 +486,18 @@ static int stack_spin(SpinTables &t)
     return pack_hops(t);
 }
 
-int sector_build_stacked(dmed_sector *s, int nup, int ndw)
+int sector_build_stacked(dmed_sector *s, int nup, int ndw, SpinCache *cache)
 {
-    if (int rc = sector_build(s, nup, ndw)) return rc;
+    if (int rc = sector_build(s, nup, ndw, cache)) return rc;
     DMED_HIP(hipStreamSynchronize(ex().stream));
-    if (int rc = stack_spin(s->dw)) return rc;
-    s->dim = s->up.dim * s->dw.dim;
+    // tables of its own: the stacked ones differ from the sector's
+    auto dw = std::make_shared<SpinTables>();
+    if (int rc = build_spin(cur_model(), 1, ndw, *dw, ex().stream)) return rc;
+    if (s->jterms)
+        if (int rc = build_pairs(cur_model(), *dw)) return rc;
+    if (int rc = stack_spin(*dw)) return rc;
+    s->dw = std::move(dw);
+    s->dim = s->up->dim * s->dw->dim;
     return 0;
 }
 

@@ -624,19 +624,19 @@ int queue_launch(SectorQueue &q, hipStream_t st)
         const int64_t n = s->dim;
         const int m = std::min(std::max(it.ncv, it.neig + 2), kQMaxM);
         SqTask &t = tasks[k];
-        t.hu_idx = s->up.hidx;
-        t.hd_idx = s->dw.hidx;
-        t.hu_val = s->up.hval;
-        t.hd_val = s->dw.hval;
-        t.du = s->up.diag;
-        t.dd = s->dw.diag;
+        t.hu_idx = s->up->hidx;
+        t.hd_idx = s->dw->hidx;
+        t.hu_val = s->up->hval;
+        t.hd_val = s->dw->hval;
+        t.du = s->up->diag;
+        t.dd = s->dw->diag;
         t.W = s->W;
-        t.impu = s->up.imp;
-        t.impd = s->dw.imp;
-        t.dup = (int32_t)s->up.dim;
-        t.ddw = (int32_t)s->dw.dim;
-        t.nhu = s->up.nhop;
-        t.nhd = s->dw.nhop;
+        t.impu = s->up->imp;
+        t.impd = s->dw->imp;
+        t.dup = (int32_t)s->up->dim;
+        t.ddw = (int32_t)s->dw->dim;
+        t.nhu = s->up->nhop;
+        t.nhd = s->dw->nhop;
         t.nimp = s->nimp;
         t.dim = (int32_t)n;
         t.neig = it.neig;

@@ -77,6 +77,7 @@ struct StateList {
 
 struct SectorCache {
     std::map<int, dmed_sector *> m;
+    SpinCache spins;                    // shared by the sectors
     ~SectorCache()
     {
         for (auto &kv : m) dmed_sector_free(kv.second);
@@ -90,7 +91,12 @@ struct SectorCache {
             return 0;
         }
         dmed_sector *s = nullptr;
-        if (int rc = dmed_sector_create(nup, ndw, &s)) return rc;
+        auto own = std::make_unique<dmed_sector>();
+        if (int rc = sector_build(own.get(), nup, ndw, &spins)) {
+            sector_release(own.get());
+            return rc;
+        }
+        s = own.release();
         m[key] = s;
         *out = s;
         return 0;
@@ -498,7 +504,7 @@ extern "C" int dmed_solve(const dmed_solve_params *p, dmed_solve_out *out)
                 break;
             }
             if ((rc = dmed_vec_create(secs[is], DMED_FP64, &r.vecs[i]))) break;
-            rc = launch_transpose((const double *)t.vecs[i]->data, T->up.dim, T->dw.dim,
+            rc = launch_transpose((const double *)t.vecs[i]->data, T->up->dim, T->dw->dim,
                                   (double *)r.vecs[i]->data, ex().stream);
         }
     }
@@ -649,7 +655,7 @@ extern "C" int dmed_solve(const dmed_solve_params *p, dmed_solve_out *out)
                             auto it = stacked_gf.find(key);
                             if (it == stacked_gf.end()) {
                                 auto sec = std::make_unique<dmed_sector>();
-                                if ((rc = sector_build_stacked(sec.get(), ju, jd))) {
+                                if ((rc = sector_build_stacked(sec.get(), ju, jd, &cache.spins))) {
                                     sector_release(sec.get());
                                     break;
                                 }
@@ -1016,7 +1022,8 @@ extern "C" int dmed_solve(const dmed_solve_params *p, dmed_solve_out *out)
                         auto it = stacked.find(key);
                         if (it == stacked.end()) {
                             auto sec = std::make_unique<dmed_sector>();
-                            if ((rc = sector_build_stacked(sec.get(), key / (ns + 1), key % (ns + 1)))) {
+                            if ((rc = sector_build_stacked(sec.get(), key / (ns + 1), key % (ns + 1),
+                                                           &cache.spins))) {
                                 sector_release(sec.get());
                                 break;
                             }
