@@ -121,12 +121,14 @@ int host_syev(int n, double *a, double *w)
     std::vector<double> Q((size_t)n * n, 0.0), v(n), p(n), q(n), e(n, 0.0);
     for (int i = 0; i < n; ++i) Q[(size_t)i * n + i] = 1.0;
     for (int k = 0; k + 2 < n; ++k) {
-        double sig = 0.0;
-        for (int i = k + 1; i < n; ++i) sig += A(i, k) * A(i, k);
+        // the entries below the sub-diagonal, summed by themselves: as sig -
+        // x0^2 entries up to 1e-8 of x0 would vanish in the rounding, and with
+        // them couplings of that size
+        double tail = 0.0;
+        for (int i = k + 2; i < n; ++i) tail += A(i, k) * A(i, k);
         const double x0 = A(k + 1, k);
-        const double tail = sig - x0 * x0;
         if (tail == 0.0) continue;                       // column already reduced
-        const double nrm = std::sqrt(sig);
+        const double nrm = std::sqrt(x0 * x0 + tail);
         const double alpha = x0 > 0 ? -nrm : nrm;
         for (int i = 0; i < n; ++i) v[i] = 0.0;
         for (int i = k + 1; i < n; ++i) v[i] = A(i, k);
