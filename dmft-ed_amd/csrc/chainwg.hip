@@ -17,8 +17,8 @@
 // (1,225), 15.4 -> 3.9 us (4,900), 17.4 -> 6.7 us (7,056).
 //
 // The recurrence and its scalars are those of the launches in krylov.hip
-// (k_hxv in Lanczos mode, k_chain_alpha, k_chain_update, k_chain_beta); only
-// the order of the reductions differs.
+// (k_hxv in Lanczos mode, k_chain_alpha, k_chain_update, k_chain_beta, k_accum);
+// only the order of the reductions differs.
 #include <algorithm>
 #include <cstdlib>
 
@@ -66,6 +66,8 @@ struct WgArgs {
     double jx, jp;
     ChainScalars *cs;
     double *alpha, *beta;
+    double *psi;                        // with psi: psi += z_k v_k, step by step
+    const double *z;
 };
 
 // LDS: the wave sums of a step's two reductions, the vector, and the hop
@@ -110,6 +112,11 @@ __global__ void __launch_bounds__(1024) k_chain_wg(const WgArgs<T> a)
     }
     __syncthreads();
     for (int it = 0; it < a.count && !cs.done; ++it) {
+        if (a.psi) {
+            const double c = a.z[cs.step] * cs.sx;
+#pragma unroll 1
+            for (int e = threadIdx.x; e < n; e += blockDim.x) a.psi[e] += c * (double)x[e];
+        }
 #pragma unroll
         for (int r = 0; r < R; ++r) y[r] = diag[r] * x[id[r] * dup + iu];
 #pragma unroll 1
@@ -245,7 +252,7 @@ WgShape wg_shape(const dmed_sector *s, int prec)
 
 template <typename T, int R>
 int launch_wg(const dmed_sector *s, const WgShape &w, void *vp, void *v, int count, ChainScalars *cs,
-              double *alpha, double *beta, hipStream_t st)
+              double *alpha, double *beta, double *psi, const double *z, hipStream_t st)
 {
     WgArgs<T> a;
     a.vp = static_cast<T *>(vp);
@@ -279,6 +286,8 @@ int launch_wg(const dmed_sector *s, const WgShape &w, void *vp, void *v, int cou
     a.cs = cs;
     a.alpha = alpha;
     a.beta = beta;
+    a.psi = psi;
+    a.z = z;
     const auto kern = s->jterms ? k_chain_wg<T, R, true> : k_chain_wg<T, R, false>;
     if (int rc = lds_attr_once((const void *)kern)) return rc;
     hipLaunchKernelGGL(kern, dim3(1), dim3(w.bs), w.lds, st, a);
@@ -288,11 +297,12 @@ int launch_wg(const dmed_sector *s, const WgShape &w, void *vp, void *v, int cou
 
 template <typename T>
 int launch_wg_r(const dmed_sector *s, const WgShape &w, void *vp, void *v, int count,
-                ChainScalars *cs, double *alpha, double *beta, hipStream_t st)
+                ChainScalars *cs, double *alpha, double *beta, double *psi, const double *z,
+                hipStream_t st)
 {
     switch (w.r) {
 #define DMED_WG(R) \
-    case R: return launch_wg<T, R>(s, w, vp, v, count, cs, alpha, beta, st);
+    case R: return launch_wg<T, R>(s, w, vp, v, count, cs, alpha, beta, psi, z, st);
         DMED_WG(1) DMED_WG(2) DMED_WG(3) DMED_WG(4) DMED_WG(5) DMED_WG(6) DMED_WG(7) DMED_WG(8)
 #undef DMED_WG
     }
@@ -304,12 +314,12 @@ int launch_wg_r(const dmed_sector *s, const WgShape &w, void *vp, void *v, int c
 bool chain_wg_takes(const dmed_sector *s, int prec) { return wg_shape(s, prec).bs > 0; }
 
 int chain_wg_steps(const dmed_sector *s, void *vp, void *v, int prec, int count, ChainScalars *cs,
-                   double *alpha, double *beta, hipStream_t st)
+                   double *alpha, double *beta, double *psi, const double *z, hipStream_t st)
 {
     const WgShape w = wg_shape(s, prec);
     if (w.bs == 0) return fail(DMED_EINVAL, "sector too large for the one-workgroup chain");
-    return prec == DMED_FP32 ? launch_wg_r<float>(s, w, vp, v, count, cs, alpha, beta, st)
-                             : launch_wg_r<double>(s, w, vp, v, count, cs, alpha, beta, st);
+    return prec == DMED_FP32 ? launch_wg_r<float>(s, w, vp, v, count, cs, alpha, beta, psi, z, st)
+                             : launch_wg_r<double>(s, w, vp, v, count, cs, alpha, beta, psi, z, st);
 }
 
 }  // namespace dmed

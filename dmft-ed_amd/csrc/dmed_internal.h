@@ -264,7 +264,7 @@ int chain_run_noalloc(const dmed_sector *s, const void *v0, int v0prec, int nlan
 constexpr int64_t kChainWgMaxDim = 8192;
 bool chain_wg_takes(const dmed_sector *s, int prec);
 int chain_wg_steps(const dmed_sector *s, void *vp, void *v, int prec, int count, ChainScalars *cs,
-                   double *alpha, double *beta, hipStream_t st);
+                   double *alpha, double *beta, double *psi, const double *z, hipStream_t st);
 int eigh_sector(const dmed_sector *s, int neig, int ncv, int maxit, double tol,
                 int dense_threshold, double *evals, dmed_vec **evecs, double *resid);
 // lowest_multiplet: the lowest level and its copies within `degen` (at most

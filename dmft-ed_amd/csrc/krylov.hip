@@ -729,8 +729,9 @@ int chain_steps(const dmed_sector *s, void *bufs[3], int prec, int count, double
     hipStream_t st = ex().stream;
     const int64_t n = s->dim;
     ChainScalars *cs = chain_scalars();
-    if (!psi && chain_wg_takes(s, prec))
-        return chain_wg_steps(s, bufs[0], bufs[1], prec, count, cs, chain_alpha(), chain_beta(), st);
+    if (chain_wg_takes(s, prec))
+        return chain_wg_steps(s, bufs[0], bufs[1], prec, count, cs, chain_alpha(), chain_beta(), psi,
+                              chain_aux(), st);
     const int nph = hxv_nparts(s, prec);
     const unsigned g = vec_grid(n);
     // the kernels of one step; no memsets, no host synchronisation

@@ -95,3 +95,23 @@ def test_small_chain_mixed_head_and_exits():
     a1, b1, _ = dmed.chain(s, v, 60)
     a2, b2, _ = dmed.chain(s, v, 60)
     assert np.array_equal(a1, a2) and np.array_equal(b1, b2)
+
+
+@pytest.mark.parametrize("norb,nbath,nup,ndw,jh", [
+    (1, 5, 3, 3, 0), (1, 7, 4, 3, 0), (1, 8, 3, 3, 0), (2, 3, 4, 4, 1), (1, 8, 4, 4, 0)])
+@pytest.mark.parametrize("prec", [dmed.FP64, dmed.MIXED])
+def test_small_ground_state(norb, nbath, nup, ndw, jh, prec):
+    """The two-pass ground state, whose second pass adds up the vector: its
+    residual is below the tolerance, on the oracle's H*v too."""
+    print(f"[small ground] norb={norb} nbath={nbath} {nup}/{ndw} jh={jh} prec={prec}", flush=True)
+    model(norb, nbath, jh)
+    s = dmed.Sector(nup, ndw)
+    e, v, res, rc = s.ground_state(prec=prec, tol=1e-11)
+    assert rc == 0 and res <= 1e-11 * max(1, abs(e))
+    x = v.download()
+    w = edref.hxv(edref.build_sector(nup, ndw), x).real
+    # 1e-11 asked for, plus the roundings of two H*v (a few ulp of ||H|| <= 60)
+    assert np.linalg.norm(w - e * x) <= 1e-11 * max(1, abs(e)) + 1e-12
+    assert abs(np.linalg.norm(x) - 1) < 1e-13
+    ev, _, _, rc = s.eigh(1, dense_threshold=16)
+    assert rc == 0 and abs(ev[0] - e) < 1e-10
