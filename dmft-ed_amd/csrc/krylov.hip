@@ -478,6 +478,29 @@ __global__ void __launch_bounds__(kVecBS) k_proj_axpy(
     if (threadIdx.x == 0) Pn[blockIdx.x] = s2;
 }
 
+// sum of np >= 1 partials, valid in every thread: each thread sums its
+// partials in index order, four loads in flight (unconditional, at clamped
+// indices)
+__device__ __forceinline__ double psum_any(const double *__restrict__ p, int np, double *red)
+{
+    __shared__ double out;
+    double s = 0.0;
+    for (int i0 = 0; i0 < np; i0 += 4 * kVecBS) {
+        double v[4];
+#pragma unroll
+        for (int k = 0; k < 4; ++k) v[k] = p[min(i0 + (int)threadIdx.x + k * kVecBS, np - 1)];
+#pragma unroll
+        for (int k = 0; k < 4; ++k)
+            if (i0 + (int)threadIdx.x + k * kVecBS < np) s += v[k];
+    }
+    s = bsum(s, red);
+    if (threadIdx.x == 0) out = s;
+    __syncthreads();
+    s = out;
+    __syncthreads();
+    return s;
+}
+
 // Lanczos three-term step of a thick-restart expansion step j (not the first
 // of a restart cycle): w -= alpha v_j + beta v_{j-1} before the full
 // Gram-Schmidt pass, with alpha = <v_j, H v_j> summed from the np partials
@@ -495,22 +518,7 @@ __global__ void __launch_bounds__(kVecBS) k_trl_local(double *__restrict__ w,
                                                       double *__restrict__ acc, int j)
 {
     __shared__ double red[16];
-    __shared__ double out;
-    // alpha: each thread sums its partials in index order, four loads in
-    // flight (unconditional, at clamped indices)
-    double s = 0.0;
-    for (int i0 = 0; i0 < np; i0 += 4 * kVecBS) {
-        double v[4];
-#pragma unroll
-        for (int k = 0; k < 4; ++k) v[k] = pa[min(i0 + (int)threadIdx.x + k * kVecBS, np - 1)];
-#pragma unroll
-        for (int k = 0; k < 4; ++k)
-            if (i0 + (int)threadIdx.x + k * kVecBS < np) s += v[k];
-    }
-    s = bsum(s, red);
-    if (threadIdx.x == 0) out = s;
-    __syncthreads();
-    const double al = out, b = *bprev;
+    const double al = psum_any(pa, np, red), b = *bprev;
     if (blockIdx.x == 0)
         for (int r = threadIdx.x; r <= j; r += blockDim.x)
             acc[r] = r == j ? al : (r == j - 1 ? b : 0.0);
@@ -519,6 +527,175 @@ __global__ void __launch_bounds__(kVecBS) k_trl_local(double *__restrict__ w,
         const double a = w[i], x = vj[i], y = vjm1[i];
         w[i] = a - al * x - b * y;
     }
+}
+
+// Two expansion steps j, j+1 that share one Gram-Schmidt pass (neither the
+// first of a restart cycle).  The three-term step leaves a remainder of
+// rounding size in the basis, so one more product can be taken before it is
+// removed: w1 = H v_j and w2 = H w1/||w1|| both take their three-term step, and
+// then one pass over the basis gives the projections of both and one removes
+// them.  The basis is read twice for two steps instead of four times (or
+// more, with the gated second passes, which a remainder of rounding size
+// never needs), and the two steps take seven launches instead of fourteen.
+// Bound by those reads of the basis.  Lowest pair of an 853,776-state sector
+// to 1e-12 (20 basis vectors): 54 -> 41 ms.
+//
+// With r the remainder of w1, |r| ~ eps |H|: alpha is off by 2 <v_j, r> and the
+// part s H r of w2 lies in the span that the pass takes off, so alpha, beta and
+// the basis are as good as from single steps as long as s |r| is small, that is
+// while no norm falls below kPairNorm times the scale of H; the host looks at
+// the norms of a cycle and takes it again with single steps otherwise.
+//
+// k_trl_first: w1 -= alpha v_j + b v_{j-1}, as k_trl_local, with the block
+// partials of ||w1||^2 in Pw.
+// k_trl_second: w2 = s y - alpha s w1 - beta v_j for y = H w1, where beta =
+// ||w1||, s = 1/beta and alpha = s^2 <w1, y> (the np partials pa).  Block 0
+// stores beta at cj[m+1] and the row of step j+1: alpha at [j+1], beta at [j].
+constexpr double kPairNorm = 1e-3;
+
+__global__ void __launch_bounds__(kVecBS) k_trl_first(double *__restrict__ w,
+                                                      const double *__restrict__ vj,
+                                                      const double *__restrict__ vjm1, int64_t n,
+                                                      const double *__restrict__ pa, int np,
+                                                      const double *__restrict__ bprev,
+                                                      double *__restrict__ acc, int j,
+                                                      double *__restrict__ Pw)
+{
+    __shared__ double red[16];
+    const double al = psum_any(pa, np, red), b = *bprev;
+    if (blockIdx.x == 0)
+        for (int r = threadIdx.x; r <= j; r += blockDim.x)
+            acc[r] = r == j ? al : (r == j - 1 ? b : 0.0);
+    double s2 = 0.0;
+    for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n;
+         i += (int64_t)gridDim.x * blockDim.x) {
+        const double a = w[i], x = vj[i], y = vjm1[i];
+        const double r = a - al * x - b * y;
+        w[i] = r;
+        s2 += r * r;
+    }
+    s2 = bsum(s2, red);
+    if (threadIdx.x == 0) Pw[blockIdx.x] = s2;
+}
+
+__global__ void __launch_bounds__(kVecBS) k_trl_second(double *__restrict__ w2,
+                                                       const double *__restrict__ w1,
+                                                       const double *__restrict__ vj, int64_t n,
+                                                       const double *__restrict__ pa, int np,
+                                                       const double *__restrict__ Pw,
+                                                       double *__restrict__ cj,
+                                                       double *__restrict__ cj1, int j, int m)
+{
+    __shared__ double red[16];
+    const double be = sqrt(psum_all(Pw, gridDim.x, red));
+    const double s = be > 0.0 ? 1.0 / be : 0.0;
+    const double al = s * s * psum_any(pa, np, red);
+    if (blockIdx.x == 0) {
+        if (threadIdx.x == 0) cj[m + 1] = be;
+        for (int r = threadIdx.x; r <= j + 1; r += blockDim.x)
+            cj1[r] = r == j + 1 ? al : (r == j ? be : 0.0);
+    }
+    const double as = al * s;
+    for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n;
+         i += (int64_t)gridDim.x * blockDim.x) {
+        const double y = w2[i], x = w1[i], z = vj[i];
+        w2[i] = s * y - as * x - be * z;
+    }
+}
+
+// Partials of the projections of w1 and w2 on the rows Y_0..Y_{ny-1},
+// V_0..V_{nv-1}: P[(2r)*gridDim.x + block] and P[(2r+1)*gridDim.x + block]; and
+// of <w1, w2> in row 2*(ny+nv).  rpb rows a block, as in k_proj_dot.
+__global__ void __launch_bounds__(kVecBS) k_proj_dot2(
+    const double *__restrict__ Y, int ny, const double *__restrict__ V, int nv,
+    const double *__restrict__ w1, const double *__restrict__ w2, int64_t n,
+    double *__restrict__ P, int rpb)
+{
+    __shared__ double red[16];
+    const int nr = ny + nv, r0 = blockIdx.y * rpb, nq = min(rpb, nr - r0);
+    const double *b[kProjRows];
+    double s1[kProjRows], s2[kProjRows], s12 = 0.0;
+#pragma unroll
+    for (int q = 0; q < kProjRows; ++q) {
+        const int r = min(r0 + q, nr - 1);
+        b[q] = r < ny ? Y + (int64_t)r * n : V + (int64_t)(r - ny) * n;
+        s1[q] = s2[q] = 0.0;
+    }
+    for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n;
+         i += (int64_t)gridDim.x * blockDim.x) {
+        const double a1 = w1[i], a2 = w2[i];
+        double x[kProjRows];
+#pragma unroll
+        for (int q = 0; q < kProjRows; ++q)
+            if (q < nq) x[q] = b[q][i];
+#pragma unroll
+        for (int q = 0; q < kProjRows; ++q)
+            if (q < nq) {
+                s1[q] += x[q] * a1;
+                s2[q] += x[q] * a2;
+            }
+        s12 += a1 * a2;
+    }
+#pragma unroll
+    for (int q = 0; q < kProjRows; ++q) {
+        if (q >= nq) break;
+        const double t1 = bsum(s1[q], red);
+        __syncthreads();
+        const double t2 = bsum(s2[q], red);
+        if (threadIdx.x == 0) {
+            P[(int64_t)(2 * (r0 + q)) * gridDim.x + blockIdx.x] = t1;
+            P[(int64_t)(2 * (r0 + q) + 1) * gridDim.x + blockIdx.x] = t2;
+        }
+        __syncthreads();
+    }
+    if (blockIdx.y == 0) {
+        s12 = bsum(s12, red);
+        if (threadIdx.x == 0) P[(int64_t)(2 * nr) * gridDim.x + blockIdx.x] = s12;
+    }
+}
+
+// v = s w1 - sum_r row_r c1_r (in place of w1) and w2 -= sum_r row_r c2_r +
+// <v', w2> v' with v' = s w1, s = 1/*beta and the coefficients from the
+// partials of k_proj_dot2 (c1 scaled by s); block partials of the new
+// ||w2||^2 in Pn.
+__global__ void __launch_bounds__(kVecBS) k_proj_axpy2(
+    const double *__restrict__ Y, int ny, const double *__restrict__ V, int nv,
+    double *__restrict__ w1, double *__restrict__ w2, int64_t n, const double *__restrict__ P,
+    const double *__restrict__ beta, double *__restrict__ Pn)
+{
+    __shared__ double red[16];
+    __shared__ double red16[16 * (kVecBS / 64)];
+    __shared__ double c[2 * kGsMaxRows + 1];
+    const int nr = ny + nv;
+    rowsums(P, 2 * nr + 1, gridDim.x, c, red16);
+    const double be = *beta, sc = be > 0.0 ? 1.0 / be : 0.0;
+    const double cab = sc * c[2 * nr];
+    double s2 = 0.0;
+    for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n;
+         i += (int64_t)gridDim.x * blockDim.x) {
+        const double a1 = sc * w1[i], a2 = w2[i];
+        double t1 = 0.0, t2 = 0.0;
+        for (int j0 = 0; j0 < nr; j0 += kProjRows) {
+            double x[kProjRows];
+#pragma unroll
+            for (int q = 0; q < kProjRows; ++q) {
+                const int j = j0 + q;
+                if (j < nr) x[q] = (j < ny ? Y + (int64_t)j * n : V + (int64_t)(j - ny) * n)[i];
+            }
+#pragma unroll
+            for (int q = 0; q < kProjRows; ++q)
+                if (j0 + q < nr) {
+                    t1 += x[q] * c[2 * (j0 + q)];
+                    t2 += x[q] * c[2 * (j0 + q) + 1];
+                }
+        }
+        w1[i] = a1 - sc * t1;
+        const double r = a2 - t2 - cab * a1;
+        w2[i] = r;
+        s2 += r * r;
+    }
+    s2 = bsum(s2, red);
+    if (threadIdx.x == 0) Pn[blockIdx.x] = s2;
 }
 
 // dst = w / ||w||, with ||w||^2 the sum of the partials p1 (after the first
@@ -1231,11 +1408,13 @@ int plain_gs(const dmed_sector *s, int maxit, double tol, double *eval, dmed_vec
 // Thick-restart Lanczos with full reorthogonalisation in a device basis, for
 // the neig lowest eigenpairs of H restricted to the orthogonal complement of
 // nl locked orthonormal vectors Y (Wu & Simon, SIAM J. Matrix Anal. Appl. 22
-// (2000) 602).  Each expansion step after the first of a restart cycle takes
-// the three-term Lanczos step, then one classical Gram-Schmidt pass against
-// Y and the basis, and a second pass when the first cancelled more than half
-// of ||w||^2; the first step of a cycle takes the two passes directly.  Ritz
-// vectors are written to X (neig contiguous device vectors).
+// (2000) 602).  The expansion steps after the first of a restart cycle take
+// the three-term Lanczos step and, two at a time, one classical Gram-Schmidt
+// pass against Y and the basis; a last odd one, and all of them once a norm
+// has come out too small for that, take a pass of their own and a second when
+// the first cancelled more than half of ||w||^2.  The first step of a cycle
+// takes the two passes directly.  Ritz vectors are written to X (neig
+// contiguous device vectors).
 int trl_run(const dmed_sector *s, int neig, int m, int maxit, double tol, const double *Y,
             int nl, uint64_t seed, double *theta_out, double *X, double *resid_out, int *used_out)
 {
@@ -1273,9 +1452,10 @@ int trl_run(const dmed_sector *s, int neig, int m, int maxit, double tol, const 
     const unsigned g = (unsigned)std::min<unsigned>(vec_grid(n), kGsGrid);
     const int nr = nl + m;
     const int nph = hxv_nparts(s, DMED_FP64);
-    if (int rc = ensure_partials((size_t)(2 * nr + 3) * g + (size_t)nph + 16)) return rc;
+    if (int rc = ensure_partials((size_t)(2 * nr + 4) * g + (size_t)nph + 16)) return rc;
     double *P1 = ex().partials, *Pn1 = P1 + (size_t)(nr + 1) * g, *P2 = Pn1 + g, *Pn2 = P2 + (size_t)nr * g;
     double *Pa = Pn2 + g;
+    double *Pw = Pa + nph;              // ||w1||^2 of a pair of steps, g values
     // classical Gram-Schmidt of w against Y[0..nl) and V[0..jmax), repeated
     // once when the first pass cancelled more than half of ||w||^2 (Daniel-
     // Gragg-Kaufman-Stewart criterion, decided on the device); the V
@@ -1309,6 +1489,28 @@ int trl_run(const dmed_sector *s, int neig, int m, int maxit, double tol, const 
         n0_last = n0;
         return 0;
     };
+    // steps j and j+1 with one Gram-Schmidt pass (k_trl_first); v_{j+1} and
+    // v_{j+2} are left in V.  Its projections take the first 2*rows + 1 rows
+    // of P1.., the norm of w2 is in Pn2.
+    auto pair = [&](int j) -> int {
+        double *vj = V + (size_t)j * n, *w1 = vj + n;
+        double *cj = dcoef + (size_t)j * ldc, *cj1 = cj + ldc;
+        if (int rc = launch_hxv(s, vj, w1, DMED_FP64, kLanczos, tcs, Pa, nullptr, st)) return rc;
+        hipLaunchKernelGGL(k_trl_first, dim3(g), dim3(kVecBS), 0, st, w1, vj, vj - n, n, Pa, nph,
+                           dcoef + (size_t)(j - 1) * ldc + m + 1, cj, j, Pw);
+        if (int rc = launch_hxv(s, w1, w, DMED_FP64, kLanczos, tcs, Pa, nullptr, st)) return rc;
+        hipLaunchKernelGGL(k_trl_second, dim3(g), dim3(kVecBS), 0, st, w, w1, vj, n, Pa, nph, Pw, cj,
+                           cj1, j, m);
+        const int rows = nl + j + 1, rpb = proj_rpb(n);
+        hipLaunchKernelGGL(k_proj_dot2, dim3(g, proj_groups(rows, rpb)), dim3(kVecBS), 0, st, Y, nl, V,
+                           j + 1, w1, w, n, P1, rpb);
+        hipLaunchKernelGGL(k_proj_axpy2, dim3(g), dim3(kVecBS), 0, st, Y, nl, V, j + 1, w1, w, n, P1,
+                           cj + m + 1, Pn2);
+        hipLaunchKernelGGL(k_normalize, dim3(g), dim3(kVecBS), 0, st, w1 + n, w, n, Pn2, Pn2, Pn2, 1,
+                           cj1 + m + 1);
+        DMED_HIP(hipGetLastError());
+        return 0;
+    };
     // dst = w/||w|| with the norm from the partials orth left; stored at nrm
     auto normalize_into = [&](double *dst, double *nrm) -> int {
         hipLaunchKernelGGL(k_normalize, dim3(g), dim3(kVecBS), 0, st, dst, w, n,
@@ -1323,17 +1525,24 @@ int trl_run(const dmed_sector *s, int neig, int m, int maxit, double tol, const 
     if (int rc = normalize_into(V, dcoef + m + 1)) return rc;
     int k = 0, used = 0;
     double beta_last = 0.0;
-    bool converged = false;
+    bool converged = false, pairs = !full;
     for (;;) {
         // expansion k..m-1 entirely on the stream; one copy of the
         // coefficients per restart
         // expansion step j > k: H v_j has, in exact arithmetic, only the
         // components alpha_j v_j and beta_{j-1} v_{j-1} in the basis; they are
-        // taken off first (k_trl_local), so the full pass that follows sees no
-        // large cancellation and its second pass seldom runs.  Step k (the
-        // arrow of the kept Ritz vectors, or the first step) goes straight to
-        // the full passes.
+        // taken off first, so the full pass that follows sees no large
+        // cancellation; two such steps share their full pass (pair), a last
+        // odd one takes its own (k_trl_local and orth).  Step k (the arrow of
+        // the kept Ritz vectors, or the first step) goes straight to the full
+        // passes.
         for (int j = k; j < m; ++j) {
+            if (pairs && j > k && j + 1 < m) {
+                if (int rc = pair(j)) return rc;
+                used += 2;
+                ++j;
+                continue;
+            }
             double *vj = V + (size_t)j * n;
             const bool local = j > k;
             if (int rc = launch_hxv(s, vj, w, DMED_FP64, local ? kLanczos : kPlain,
@@ -1352,6 +1561,24 @@ int trl_run(const dmed_sector *s, int neig, int m, int maxit, double tol, const 
         DMED_HIP(hipMemcpyAsync(hc.data() + (size_t)k * ldc, dcoef + (size_t)k * ldc,
                                 (size_t)(m - k) * ldc * 8, hipMemcpyDeviceToHost, st));
         DMED_HIP(hipStreamSynchronize(st));
+        if (pairs) {
+            // a norm far below the scale of H: the pairs' remainder is no
+            // longer of rounding size against it (an invariant subspace, or
+            // nearly one).  Columns 0..k of the basis are as they were, so the
+            // cycle is taken again with single steps.
+            double hn = 0.0, bmin = INFINITY;
+            for (int j = k; j < m; ++j) {
+                const double *c1 = hc.data() + (size_t)j * ldc, bn = c1[m + 1];
+                hn = std::max(hn, std::max(fabs(c1[j]), bn));
+                if (j > k && !(bn >= bmin)) bmin = bn;   // also a NaN
+            }
+            for (int q = 0; q < k; ++q) hn = std::max(hn, fabs(T[(size_t)q * m + q]));
+            if (!(bmin > kPairNorm * hn)) {
+                pairs = false;
+                used -= m - k;
+                continue;
+            }
+        }
         for (int j = k; j < m; ++j) {
             const double *c1 = hc.data() + (size_t)j * ldc;
             for (int q = 0; q <= j; ++q) {
