@@ -279,6 +279,10 @@ int eigh_sector_ex(const dmed_sector *s, int neig, int ncv, int maxit, double to
 int ground_state(const dmed_sector *s, int prec, int maxit, double tol, double *eval,
                  dmed_vec **evec, double *resid);
 
+// smallest norm, against the scale of H, at which two steps of a thick-restart
+// Lanczos run share a Gram-Schmidt pass (k_trl_first)
+constexpr double kPairNorm = 1e-3;
+
 // --------------------------------------------- persistent sector queue
 // Small Krylov sectors of a batched solve, diagonalised by one launch of a
 // persistent work-queue kernel (sectorq.hip): each workgroup takes a sector

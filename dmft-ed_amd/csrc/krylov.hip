@@ -551,8 +551,6 @@ __global__ void __launch_bounds__(kVecBS) k_trl_local(double *__restrict__ w,
 // k_trl_second: w2 = s y - alpha s w1 - beta v_j for y = H w1, where beta =
 // ||w1||, s = 1/beta and alpha = s^2 <w1, y> (the np partials pa).  Block 0
 // stores beta at cj[m+1] and the row of step j+1: alpha at [j+1], beta at [j].
-constexpr double kPairNorm = 1e-3;
-
 __global__ void __launch_bounds__(kVecBS) k_trl_first(double *__restrict__ w,
                                                       const double *__restrict__ vj,
                                                       const double *__restrict__ vjm1, int64_t n,
