@@ -117,6 +117,7 @@ namespace dmed {
 
 // ------------------------------------------------------------- context
 constexpr int kScalCap = 4096;
+constexpr int kChainMax = (kScalCap - 16) / 3;   // steps of a chain
 
 // An execution context: one HIP stream with its own reduction scratch,
 // device scalars (Lanczos chain state) and grow-only work buffers.  The
@@ -136,7 +137,9 @@ constexpr int kSlotMid = 10;            // intermediate vector of a two-operator
 constexpr int kSlotGf = 11;             // coefficients, frequencies and results of a G sum
 constexpr int kSlotChainLo = 12;        // 12..14: FP32 tail of a mixed chain
 constexpr int kSlotDense = 15;          // matrices of a dense batch
-constexpr int kExecSlots = 16;
+constexpr int kSlotBatchVec = 16;       // start vectors of a chain batch
+constexpr int kSlotChainBatch = 17;     // descriptors and coefficients of a chain batch
+constexpr int kExecSlots = 18;
 constexpr int kMixedHead = 32;          // FP64 steps at the head of a mixed chain
 
 struct Exec {
@@ -265,6 +268,16 @@ constexpr int64_t kChainWgMaxDim = 8192;
 bool chain_wg_takes(const dmed_sector *s, int prec);
 int chain_wg_steps(const dmed_sector *s, void *vp, void *v, int prec, int count, ChainScalars *cs,
                    double *alpha, double *beta, double *psi, const double *z, hipStream_t st);
+// whole FP64 chains of small sectors, all in one launch; alpha and beta (nlanc
+// each) are 0 past a chain's end, the start vectors stay as they are
+struct ChainBatchItem {
+    const dmed_sector *s;
+    void *v;
+    int nlanc;
+    double *alpha, *beta;
+};
+bool chain_batch_takes(const dmed_sector *s, int nlanc);
+int chain_batch_run(std::vector<ChainBatchItem> &items, double threshold);
 int eigh_sector(const dmed_sector *s, int neig, int ncv, int maxit, double tol,
                 int dense_threshold, double *evals, dmed_vec **evecs, double *resid);
 // lowest_multiplet: the lowest level and its copies within `degen` (at most

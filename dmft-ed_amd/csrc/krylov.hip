@@ -851,7 +851,6 @@ ChainScalars *chain_scalars() { return reinterpret_cast<ChainScalars *>(ex().dsc
 double *chain_alpha() { return ex().dscal + 16; }
 double *chain_beta() { return ex().dscal + 16 + (kScalCap - 16) / 3; }
 double *chain_aux() { return ex().dscal + 16 + 2 * ((kScalCap - 16) / 3); }
-constexpr int kChainMax = (kScalCap - 16) / 3;
 
 // Chain on three rotated work vectors bufs = {v_prev, v, w}; bufs[1] holds
 // the (unnormalised) start vector.  chain_init normalises it through the

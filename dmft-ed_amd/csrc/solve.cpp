@@ -222,6 +222,47 @@ double now()
     return std::chrono::duration<double>(std::chrono::steady_clock::now().time_since_epoch()).count();
 }
 
+// Start vectors of the chains that one launch takes together (chain_batch_run)
+// and what it does with them: the tasks of a phase write their vectors into
+// one slab, run() then takes all of them.  A chain without a place (too large
+// for one workgroup, another precision, slab full) is run by its task.
+constexpr size_t kBatchVecBytes = (size_t)64 << 20;
+struct ChainPhase {
+    struct Ref {
+        const dmed_sector *s = nullptr;
+        std::vector<double> *al = nullptr, *bl = nullptr;
+        size_t off = SIZE_MAX;              // of the start vector in the slab
+        bool ready = false;                 // vector written, coefficients wanted
+    };
+    std::vector<Ref> refs;
+    char *slab = nullptr;
+    explicit ChainPhase(size_t n) : refs(n) {}
+    // before the tasks run; nlanc(t) <= 0 leaves task t out
+    int plan(bool on, const std::function<Ref(size_t)> &ref, const std::function<int(size_t)> &nlanc)
+    {
+        size_t total = 0;
+        for (size_t t = 0; t < refs.size(); ++t) {
+            refs[t] = ref(t);
+            const size_t bytes = ((size_t)refs[t].s->dim * 8 + 255) / 256 * 256;
+            if (!on || !chain_batch_takes(refs[t].s, nlanc(t)) || total + bytes > kBatchVecBytes)
+                continue;
+            refs[t].off = total;
+            total += bytes;
+        }
+        return total ? exec_buf(ex(), kSlotBatchVec, total, (void **)&slab) : 0;
+    }
+    // where task t puts its start vector, null: in a buffer of its own
+    void *place(int t) { return refs[t].off == SIZE_MAX ? nullptr : slab + refs[t].off; }
+    int run()
+    {
+        std::vector<ChainBatchItem> items;
+        for (Ref &r : refs)
+            if (r.ready)
+                items.push_back({r.s, slab + r.off, (int)r.al->size(), r.al->data(), r.bl->data()});
+        return chain_batch_run(items, 1e-13);
+    }
+};
+
 }  // namespace
 
 // In-place inverse of a small complex n x n matrix (row-major), Gauss-Jordan
@@ -667,12 +708,19 @@ extern "C" int dmed_solve(const dmed_solve_params *p, dmed_solve_out *out)
                         chains.push_back(std::move(ch));
                     }
                 }
+    const bool batch = p->prec_gf == DMED_FP64;
+    ChainPhase gph(chains.size());
+    if (!rc)
+        rc = gph.plan(
+            batch, [&](size_t t) { return ChainPhase::Ref{chains[t].J, &chains[t].al, &chains[t].bl}; },
+            [&](size_t t) { return chains[t].nlanc; });
     auto run_chain = [&](int t) {
         Chain &ch = chains[t];
         const State &st = sl.items[ch.state];
-        // start vector in a reusable buffer of the calling context
-        dmed_vec v{ch.J, DMED_FP64, ch.J->dim, nullptr};
-        if ((ch.rc = exec_buf(ex(), kSlotStart, std::max<int64_t>(ch.J->dim, 1) * 8, &v.data))) {
+        // start vector in the slab of the phase or a reusable buffer of the
+        // calling context
+        dmed_vec v{ch.J, DMED_FP64, ch.J->dim, gph.place(t)};
+        if (!v.data && (ch.rc = exec_buf(ex(), kSlotStart, std::max<int64_t>(ch.J->dim, 1) * 8, &v.data))) {
             ch.err = dmed_last_error();
             return;
         }
@@ -713,14 +761,18 @@ extern "C" int dmed_solve(const dmed_solve_params *p, dmed_solve_out *out)
             ch.al.assign(ch.nlanc, 0.0);
             ch.bl.assign(ch.nlanc, 0.0);
             int nsteps = 0;
-            ch.rc = chain_run(ch.J, v.data, DMED_FP64, ch.nlanc, p->prec_gf, 1e-13, ch.al.data(),
-                              ch.bl.data(), &nsteps, p->gf_fp64_head);
+            if (gph.place(t))
+                gph.refs[t].ready = true;
+            else
+                ch.rc = chain_run(ch.J, v.data, DMED_FP64, ch.nlanc, p->prec_gf, 1e-13,
+                                  ch.al.data(), ch.bl.data(), &nsteps, p->gf_fp64_head);
         }
         if (ch.rc) ch.err = dmed_last_error();
     };
     if (!rc) rc = run_tasks(p->batched, (int)chains.size(), run_chain);
     for (auto &ch : chains)
         if (!rc && ch.rc) rc = fail(ch.rc, ch.err);
+    if (!rc) rc = gph.run();
     for (auto &kv : stacked_gf) dmed_sector_free(kv.second);
     // full orbital matrices G[s][a][b] (hybrid bath), interleaved complex
     std::vector<double> gfm(offdiag ? 2 * (size_t)nspin * norb * norb * lm : 0),
@@ -906,29 +958,41 @@ extern "C" int dmed_solve(const dmed_solve_params *p, dmed_solve_out *out)
                 t.row = row;
                 tasks.push_back(std::move(t));
             }
+        for (auto &t : tasks)
+            t.nlanc = (int)std::min<int64_t>(sl.items[t.state].vec->sec->dim, ngf);
+        ChainPhase ph(tasks.size());
+        rc = ph.plan(
+            batch,
+            [&](size_t t) {
+                return ChainPhase::Ref{sl.items[tasks[t].state].vec->sec, &tasks[t].al, &tasks[t].bl};
+            },
+            [&](size_t t) { return tasks[t].nlanc; });
         auto run_chi = [&](int t) {
             ChiTask &ck = tasks[t];
             const State &st = sl.items[ck.state];
             const dmed_sector *S = st.vec->sec;
-            dmed_vec v{S, DMED_FP64, S->dim, nullptr};
-            if ((ck.rc = exec_buf(ex(), kSlotStart, std::max<int64_t>(S->dim, 1) * 8, &v.data))) {
+            dmed_vec v{S, DMED_FP64, S->dim, ph.place(t)};
+            if (!v.data && (ck.rc = exec_buf(ex(), kSlotStart, std::max<int64_t>(S->dim, 1) * 8, &v.data))) {
                 ck.err = dmed_last_error();
                 return;
             }
             ck.rc = dmed_apply_sz(st.vec, ck.row < norb ? ck.row : -1, &v, &ck.norm2);
             if (!ck.rc && ck.norm2 > 0.0) {
-                ck.nlanc = (int)std::min<int64_t>(S->dim, ngf);
                 ck.al.assign(ck.nlanc, 0.0);
                 ck.bl.assign(ck.nlanc, 0.0);
                 int nsteps = 0;
-                ck.rc = chain_run(S, v.data, DMED_FP64, ck.nlanc, p->prec_gf, 1e-13, ck.al.data(),
-                                  ck.bl.data(), &nsteps, p->gf_fp64_head);
+                if (ph.place(t))
+                    ph.refs[t].ready = true;
+                else
+                    ck.rc = chain_run(S, v.data, DMED_FP64, ck.nlanc, p->prec_gf, 1e-13,
+                                      ck.al.data(), ck.bl.data(), &nsteps, p->gf_fp64_head);
             }
             if (ck.rc) ck.err = dmed_last_error();
         };
-        rc = run_tasks(p->batched, (int)tasks.size(), run_chi);
+        if (!rc) rc = run_tasks(p->batched, (int)tasks.size(), run_chi);
         for (auto &ck : tasks)
             if (!rc && ck.rc) rc = fail(ck.rc, ck.err);
+        if (!rc) rc = ph.run();
         if (!rc) {
             std::vector<ChiTerm> terms;
             for (auto &ck : tasks) {
@@ -1056,12 +1120,20 @@ extern "C" int dmed_solve(const dmed_solve_params *p, dmed_solve_out *out)
                 dt.push_back(std::move(t));
             }
         }
+        for (auto &t : dt)
+            t.nlanc = (int)std::min<int64_t>(
+                t.kind == kStacked ? sl.items[t.state].vec->sec->dim : t.S->dim, ngf);
+        ChainPhase ph(dt.size());
+        if (!rc)
+            rc = ph.plan(
+                batch, [&](size_t t) { return ChainPhase::Ref{dt[t].S, &dt[t].al, &dt[t].bl}; },
+                [&](size_t t) { return dt[t].nlanc; });
         auto run_dchi = [&](int t) {
             DTask &dk = dt[t];
             const State &st = sl.items[dk.state];
             const dmed_sector *I = st.vec->sec;
-            void *buf = nullptr;
-            if ((dk.rc = exec_buf(ex(), kSlotStart, std::max<int64_t>(dk.S->dim, 1) * 8, &buf))) {
+            void *buf = ph.place(t);
+            if (!buf && (dk.rc = exec_buf(ex(), kSlotStart, std::max<int64_t>(dk.S->dim, 1) * 8, &buf))) {
                 dk.err = dmed_last_error();
                 return;
             }
@@ -1086,18 +1158,21 @@ extern "C" int dmed_solve(const dmed_solve_params *p, dmed_solve_out *out)
                 if (!dk.rc) dk.rc = dmed_apply_op(&mid, dk.b + 1 + dk.spin * ns, 1, dk.S, &out, &dk.norm2);
             }
             if (!dk.rc && dk.norm2 > 0.0) {
-                dk.nlanc = (int)std::min<int64_t>(dk.kind == kStacked ? I->dim : dk.S->dim, ngf);
                 dk.al.assign(dk.nlanc, 0.0);
                 dk.bl.assign(dk.nlanc, 0.0);
                 int nsteps = 0;
-                dk.rc = chain_run(dk.S, buf, DMED_FP64, dk.nlanc, p->prec_gf, 1e-13, dk.al.data(),
-                                  dk.bl.data(), &nsteps, p->gf_fp64_head);
+                if (ph.place(t))
+                    ph.refs[t].ready = true;
+                else
+                    dk.rc = chain_run(dk.S, buf, DMED_FP64, dk.nlanc, p->prec_gf, 1e-13,
+                                      dk.al.data(), dk.bl.data(), &nsteps, p->gf_fp64_head);
             }
             if (dk.rc) dk.err = dmed_last_error();
         };
         if (!rc) rc = run_tasks(p->batched, (int)dt.size(), run_dchi);
         for (auto &dk : dt)
             if (!rc && dk.rc) rc = fail(dk.rc, dk.err);
+        if (!rc) rc = ph.run();
         for (auto &kv : stacked) dmed_sector_free(kv.second);
         if (!rc) {
             const size_t nab = (size_t)norb * norb;

@@ -115,3 +115,25 @@ def test_small_ground_state(norb, nbath, nup, ndw, jh, prec):
     assert abs(np.linalg.norm(x) - 1) < 1e-13
     ev, _, _, rc = s.eigh(1, dense_threshold=16)
     assert rc == 0 and abs(ev[0] - e) < 1e-10
+
+
+@pytest.mark.parametrize("norb,nbath,jh,nst,chi", [(1, 7, 0, 1, 0), (1, 8, 0, 8, 0), (2, 3, 1, 6, 1), (2, 2, 0, 24, 1), (1, 3, 0, 4, 0)])
+@pytest.mark.parametrize("batched", [0, 1])
+def test_chain_batch_of_a_solve(norb, nbath, jh, nst, chi, batched):
+    """The chains of a solve in one launch against the same chains one by one
+    (the mixed form with every step in its FP64 head takes that way): one to
+    eight columns per lane, stacked sectors beside plain ones, chains longer
+    than their sector."""
+    print(f"[chain batch] {norb} {nbath} jh={jh} nst={nst} chi={chi} batched={batched}", flush=True)
+    ns = model(norb, nbath, jh)
+    kw = dict(lanc_nstates_sector=2, lanc_nstates_total=nst, lmats=64, lreal=64, beta=20.0, eps=0.1,
+              ltau=40, chi_spin=chi, chi_dens=chi, lanc_ngfiter=100, batched=batched)
+    a = dmed.solve(norb, 1, ns, dmed.default_params(prec_gf=dmed.FP64, **kw))
+    ns = model(norb, nbath, jh)
+    b = dmed.solve(norb, 1, ns, dmed.default_params(prec_gf=dmed.MIXED, gf_fp64_head=100, **kw))
+    assert a["nstates"] == b["nstates"] and abs(a["egs"] - b["egs"]) < 1e-10
+    # the bars of the solve against the oracle on the same quantities
+    keys = ["gmats"] + [k for k in a if chi and k.endswith(("chi_iv", "chi_tau"))]
+    for k in keys:
+        x, y = np.asarray(a[k]), np.asarray(b[k])
+        assert np.abs(x - y).max() <= 1e-8 * max(1, np.abs(y).max()), k
