@@ -213,7 +213,7 @@ __global__ void __launch_bounds__(1024) k_hxv(const HxvArgs<T> a)
 // (in bounds) and are never stored: the inner loops carry no per-row branch,
 // so all loads of a hop step are in flight before the first is used.
 // Summation order per row: down hops in table order, up hops in table order,
-// then the diagonal -- the same for every (BS, RPT) and grid, so the launch
+// the orbital pairs, then the diagonal -- the same for every (BS, RPT) and grid, so the launch
 // shape never changes y.  In Lanczos mode each column's <x, y> is reduced on
 // its own and stored at PARTIALS[c]: alpha does not depend on the grid either.
 // Address arithmetic bounds the hop loops as much as the loads do, so a lane's
@@ -232,15 +232,29 @@ __global__ void __launch_bounds__(1024) k_hxv(const HxvArgs<T> a)
 constexpr int kColScBytes = 256 * 8, kColHeadBytes = kColScBytes + 24 * 8 + 64;
 static_assert(kColHeadBytes % 256 == 0, "the column starts on a DMA boundary");
 
-template <typename T, int MODE, int BS, int RPT, int HALVES = 1>
+// Spin exchange and pair hopping in the column kernel (JT): a pair of orbitals
+// takes a column to at most one other (exchange and pair hopping ask for
+// opposite occupations), the same for all its rows.  Most pairs take a column
+// nowhere and are skipped by the whole workgroup; of the rest the rows whose
+// own hop exists gather from the other column.  Three orbitals, D = 853,776,
+// FP64: tile kernel 34.8 us, here 13 us (without the pairs 7.8 us); a Lanczos
+// step at D = 4.1e7: 2.10 -> 0.96 ms.
+struct ColPairs {
+    const int32_t *ju, *jd;
+    int32_t norb;
+    double jx, jp;
+};
+
+template <typename T, int MODE, int BS, int RPT, int HALVES = 1, bool JT = false>
 __global__ void __launch_bounds__(BS, HALVES == 2 ? 2 * BS / 256 : 1) k_hxv_col(
     const T *__restrict__ X, T *__restrict__ Y, int32_t dup, int32_t ddw, int32_t nhu, int32_t nhd,
     int32_t nimp, int32_t ncoef, const uint32_t *__restrict__ HU, const double *__restrict__ COEF,
     const int32_t *__restrict__ HDI, const double *__restrict__ HDV, const double *__restrict__ DU,
     const double *__restrict__ DD, const uint8_t *__restrict__ IMPU, const uint8_t *__restrict__ IMPD,
     const double *__restrict__ WTAB, int32_t dma16, const ChainScalars *__restrict__ CS,
-    double *__restrict__ PARTIALS)
+    double *__restrict__ PARTIALS, const ColPairs J)
 {
+    static_assert(!JT || HALVES == 1, "pairs: one-pass form only");
     // LDS: signed coefficients, the impurity diagonal and reduction buffers at
     // fixed offsets, then the column
     extern __shared__ __align__(16) unsigned char smem[];
@@ -405,6 +419,26 @@ __global__ void __launch_bounds__(BS, HALVES == 2 ? 2 * BS / 256 : 1) k_hxv_col(
 #pragma unroll
                 for (int r = 0; r < RPT; ++r) acc[r] += sc[w[r] >> 24] * col[w[r] & 0xffffffu];
             }
+            if constexpr (JT) {
+                for (int pa = 0; pa < J.norb; ++pa)
+                    for (int pb = 0; pb < J.norb; ++pb) {
+                        if (pa == pb) continue;
+                        const int32_t wx = J.jd[(int64_t)(pb * J.norb + pa) * ddw + c];
+                        const int32_t wp = J.jd[(int64_t)(pa * J.norb + pb) * ddw + c];
+                        const int32_t wd = wx >= 0 ? wx : wp;
+                        if (wd < 0) continue;
+                        const double cd = ((wd & 1) ? -1.0 : 1.0) * (wx >= 0 ? J.jx : J.jp);
+                        const T *xj = X + (int64_t)(wd >> 1) * dup;
+                        const int32_t *ju = J.ju + (int64_t)(pa * J.norb + pb) * dup;
+                        int32_t wu[RPT];
+#pragma unroll
+                        for (int r = 0; r < RPT; ++r) wu[r] = at(ju, row(r));
+#pragma unroll
+                        for (int r = 0; r < RPT; ++r)
+                            if (wu[r] >= 0)
+                                acc[r] += (T)((wu[r] & 1) ? -cd : cd) * at(xj, (uint32_t)wu[r] >> 1);
+                    }
+            }
             // 4. diagonal last, with the lane's own x from LDS
 #pragma unroll
             for (int r = 0; r < RPT; ++r) {
@@ -473,7 +507,7 @@ static bool use_col_kernel(const dmed_sector *s, int prec)
     const Context &c = ctx();
     const size_t esz = prec == DMED_FP32 ? 4 : 8;
     const int64_t dup = s->up->dim;
-    return !s->jterms && s->up->packed && s->up->ncoef <= 128 && s->nimp <= 8 && dup >= 512 &&
+    return s->up->packed && s->up->ncoef <= 128 && s->nimp <= 8 && dup >= 512 &&
            col_rpt(s, prec, 1024) > 0 && col_lds_bytes(dup, esz) + 2048 <= c.lds_max &&
            s->dw->dim >= 64;
 }
@@ -509,9 +543,10 @@ int lds_attr_once(const void *kern)
 
 // Column-kernel instantiations: 1024 lanes with 1..13 (FP64) or 1..16 (FP32)
 // rows per lane, 512 and 256 lanes with 1..8; the two-half form (HALVES = 2)
-// for 1024 lanes and at least 4 rows per lane.  f(kernel pointer) is called
-// with the instantiation for (bs, rpt, halves); false if there is none.
-template <typename T, int MODE, int BS, int H, typename F>
+// for 1024 lanes and at least 4 rows per lane, without orbital pairs (jt).
+// f(kernel pointer) is called with the instantiation for (bs, rpt, halves, jt);
+// false if there is none.
+template <typename T, int MODE, int BS, int H, bool JT, typename F>
 static bool col_dispatch_bs(int rpt, F &&f)
 {
     switch (rpt) {
@@ -519,7 +554,7 @@ static bool col_dispatch_bs(int rpt, F &&f)
     case R:                                                                        \
         if constexpr (R <= (BS == 1024 ? (sizeof(T) == 4 ? 16 : 13) : 8) &&        \
                       (H == 1 || (BS == 1024 && R >= 4))) {                        \
-            f(k_hxv_col<T, MODE, BS, R, H>);                                       \
+            f(k_hxv_col<T, MODE, BS, R, H, JT>);                                   \
             return true;                                                           \
         }                                                                          \
         return false;
@@ -531,16 +566,25 @@ static bool col_dispatch_bs(int rpt, F &&f)
     }
 }
 
-template <typename T, int MODE, typename F>
-static bool col_dispatch(int bs, int rpt, bool halves, F &&f)
+template <typename T, int MODE, bool JT, typename F>
+static bool col_dispatch_j(int bs, int rpt, bool halves, F &&f)
 {
-    if (bs == 1024)
-        return halves ? col_dispatch_bs<T, MODE, 1024, 2>(rpt, f)
-                      : col_dispatch_bs<T, MODE, 1024, 1>(rpt, f);
-    if (halves) return false;
-    if (bs == 512) return col_dispatch_bs<T, MODE, 512, 1>(rpt, f);
-    if (bs == 256) return col_dispatch_bs<T, MODE, 256, 1>(rpt, f);
+    if (halves) {
+        if constexpr (!JT)
+            if (bs == 1024) return col_dispatch_bs<T, MODE, 1024, 2, false>(rpt, f);
+        return false;
+    }
+    if (bs == 1024) return col_dispatch_bs<T, MODE, 1024, 1, JT>(rpt, f);
+    if (bs == 512) return col_dispatch_bs<T, MODE, 512, 1, JT>(rpt, f);
+    if (bs == 256) return col_dispatch_bs<T, MODE, 256, 1, JT>(rpt, f);
     return false;
+}
+
+template <typename T, int MODE, typename F>
+static bool col_dispatch(int bs, int rpt, bool halves, bool jt, F &&f)
+{
+    return jt ? col_dispatch_j<T, MODE, true>(bs, rpt, halves, f)
+              : col_dispatch_j<T, MODE, false>(bs, rpt, halves, f);
 }
 
 // DMED_COL_HALVES=0 keeps the column kernel to its one-pass form
@@ -556,10 +600,10 @@ static bool halves_enabled()
 // workgroups of (bs, rpt, halves) per CU that registers and LDS allow; 0
 // when there is no such instantiation
 template <typename T>
-static int col_fit_per_cu(int bs, int rpt, bool halves, size_t shmem)
+static int col_fit_per_cu(int bs, int rpt, bool halves, bool jt, size_t shmem)
 {
     int nb = 1;
-    const bool ok = col_dispatch<T, kLanczos>(bs, rpt, halves, [&](auto kern) {
+    const bool ok = col_dispatch<T, kLanczos>(bs, rpt, halves, jt, [&](auto kern) {
         if (lds_attr_once((const void *)kern) != 0 ||
             hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, (const void *)kern, bs, shmem) !=
                 hipSuccess)
@@ -579,8 +623,9 @@ static ColFit col_fit(const dmed_sector *s, int prec, int bs)
 {
     // the occupancy query is the same for every sector of this shape: keep it
     static std::mutex mu;
-    static std::map<std::tuple<int64_t, int, int>, ColFit> memo;
-    const auto key = std::make_tuple(s->up->dim, prec == DMED_FP32 ? 1 : 0, bs);
+    static std::map<std::tuple<int64_t, int, int, bool>, ColFit> memo;
+    const bool jt = s->jterms != 0;
+    const auto key = std::make_tuple(s->up->dim, prec == DMED_FP32 ? 1 : 0, bs, jt);
     {
         std::lock_guard<std::mutex> lk(mu);
         auto it = memo.find(key);
@@ -593,11 +638,11 @@ static ColFit col_fit(const dmed_sector *s, int prec, int bs)
         f.one = 0;
     } else {
         const bool f32 = prec == DMED_FP32;
-        f.one = std::max(1, f32 ? col_fit_per_cu<float>(bs, rpt, false, shmem)
-                                : col_fit_per_cu<double>(bs, rpt, false, shmem));
+        f.one = std::max(1, f32 ? col_fit_per_cu<float>(bs, rpt, false, jt, shmem)
+                                : col_fit_per_cu<double>(bs, rpt, false, jt, shmem));
         if (halves_enabled() && bs == 1024)
-            f.two = f32 ? col_fit_per_cu<float>(bs, rpt, true, shmem)
-                        : col_fit_per_cu<double>(bs, rpt, true, shmem);
+            f.two = f32 ? col_fit_per_cu<float>(bs, rpt, true, jt, shmem)
+                        : col_fit_per_cu<double>(bs, rpt, true, jt, shmem);
     }
     std::lock_guard<std::mutex> lk(mu);
     memo[key] = f;
@@ -725,7 +770,7 @@ static int launch_col(const dmed_sector *s, const void *x, void *y, ChainScalars
     // 16-byte DMA granules need every column start 16-byte aligned
     const int dma16 = ((uintptr_t)x % 16 == 0) && ((size_t)dup * sizeof(T)) % 16 == 0;
     int rc = 0;
-    const bool ok = col_dispatch<T, MODE>(c.bs, c.rpt, c.halves, [&](auto kern) {
+    const bool ok = col_dispatch<T, MODE>(c.bs, c.rpt, c.halves, s->jterms != 0, [&](auto kern) {
         rc = lds_attr_once((const void *)kern);
         if (rc) return;
         hipLaunchKernelGGL(kern, dim3(c.grid), dim3(c.bs), shmem, st, static_cast<const T *>(x),
@@ -733,7 +778,8 @@ static int launch_col(const dmed_sector *s, const void *x, void *y, ChainScalars
                            (int32_t)s->up->nhop, (int32_t)s->dw->nhop, (int32_t)s->nimp,
                            (int32_t)s->up->ncoef, s->up->hpk, s->up->coef, s->dw->hidx, s->dw->hval,
                            s->up->diag, s->dw->diag, s->up->imp, s->dw->imp, s->W, (int32_t)dma16,
-                           (const ChainScalars *)cs, partials);
+                           (const ChainScalars *)cs, partials,
+                           ColPairs{s->up->ipair, s->dw->ipair, s->norb, s->jx, s->jp});
     });
     if (!ok) return fail(DMED_EINVAL, "column kernel: unsupported rows per lane");
     if (rc) return rc;
