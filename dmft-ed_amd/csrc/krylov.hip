@@ -134,6 +134,29 @@ __global__ void __launch_bounds__(1024) k_chain_alpha(const double *__restrict__
     }
 }
 
+// sum of np >= 1 partials, valid in every thread: each thread sums its
+// partials in index order, four loads in flight (unconditional, at clamped
+// indices)
+__device__ __forceinline__ double psum_any(const double *__restrict__ p, int np, double *red)
+{
+    __shared__ double out;
+    double s = 0.0;
+    for (int i0 = 0; i0 < np; i0 += 4 * kVecBS) {
+        double v[4];
+#pragma unroll
+        for (int k = 0; k < 4; ++k) v[k] = p[min(i0 + (int)threadIdx.x + k * kVecBS, np - 1)];
+#pragma unroll
+        for (int k = 0; k < 4; ++k)
+            if (i0 + (int)threadIdx.x + k * kVecBS < np) s += v[k];
+    }
+    s = bsum(s, red);
+    if (threadIdx.x == 0) out = s;
+    __syncthreads();
+    s = out;
+    __syncthreads();
+    return s;
+}
+
 // 16-byte vectors of T
 template <typename T> struct Vec16;
 template <> struct Vec16<double> { using type = double2; };
@@ -144,16 +167,34 @@ template <> struct Vec16<float> { using type = float4; };
 // Each thread takes the elements i = tid + k*stride in increasing order, as a
 // plain grid-stride loop would, with four of them loaded before the first is
 // used; the partial sums (hence beta) do not depend on that grouping.
+// np > 0: the np partials pa of <v, y> are summed here, by every block, instead
+// of by k_chain_alpha (block 0 stores alpha).  Up to kAlphaFold of them that
+// costs less than the launch: a step at D = 853,776 takes 29.0 us, not 29.9; past it the
+// re-reads by all blocks cost more.
+constexpr int kAlphaFold = 4096;
 template <typename T>
 __global__ void __launch_bounds__(kVecBS) k_chain_update(T *__restrict__ w, const T *__restrict__ v,
                                                          const T *__restrict__ vp, int64_t n,
-                                                         const ChainScalars *cs,
-                                                         double *__restrict__ partials)
+                                                         ChainScalars *cs,
+                                                         double *__restrict__ partials,
+                                                         const double *__restrict__ pa, int np,
+                                                         double *__restrict__ alpha)
 {
     constexpr int U = 4;
     __shared__ double red[16];
     if (cs->done) return;
-    const double ca = cs->alpha * cs->sx, cb = cs->b * cs->svp;
+    const double cb = cs->b * cs->svp;
+    double al;
+    if (np > 0) {
+        al = cs->sx * (psum_any(pa, np, red) - cb * cs->q);      // as k_chain_alpha
+        if (blockIdx.x == 0 && threadIdx.x == 0) {
+            cs->alpha = al;
+            alpha[cs->step] = al;
+        }
+    } else {
+        al = cs->alpha;
+    }
+    const double ca = al * cs->sx;
     double s1 = 0.0, s2 = 0.0;
     const int64_t stride = (int64_t)gridDim.x * blockDim.x;
     for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += U * stride) {
@@ -476,29 +517,6 @@ __global__ void __launch_bounds__(kVecBS) k_proj_axpy(
     }
     s2 = bsum(s2, red);
     if (threadIdx.x == 0) Pn[blockIdx.x] = s2;
-}
-
-// sum of np >= 1 partials, valid in every thread: each thread sums its
-// partials in index order, four loads in flight (unconditional, at clamped
-// indices)
-__device__ __forceinline__ double psum_any(const double *__restrict__ p, int np, double *red)
-{
-    __shared__ double out;
-    double s = 0.0;
-    for (int i0 = 0; i0 < np; i0 += 4 * kVecBS) {
-        double v[4];
-#pragma unroll
-        for (int k = 0; k < 4; ++k) v[k] = p[min(i0 + (int)threadIdx.x + k * kVecBS, np - 1)];
-#pragma unroll
-        for (int k = 0; k < 4; ++k)
-            if (i0 + (int)threadIdx.x + k * kVecBS < np) s += v[k];
-    }
-    s = bsum(s, red);
-    if (threadIdx.x == 0) out = s;
-    __syncthreads();
-    s = out;
-    __syncthreads();
-    return s;
 }
 
 // Lanczos three-term step of a thick-restart expansion step j (not the first
@@ -908,6 +926,7 @@ int chain_steps(const dmed_sector *s, void *bufs[3], int prec, int count, double
                               chain_aux(), st);
     const int nph = hxv_nparts(s, prec);
     const unsigned g = vec_grid(n);
+    double *pu = partials + nph;        // the update's sums, beside those of H*v
     // the kernels of one step; no memsets, no host synchronisation
     auto one = [&](void *vp, void *v, void *w) -> int {
         if (psi) {
@@ -920,16 +939,17 @@ int chain_steps(const dmed_sector *s, void *bufs[3], int prec, int count, double
         }
         if (int rc = launch_hxv(s, v, w, prec, kLanczos, cs, partials, nullptr, st))
             return rc;
-        hipLaunchKernelGGL(k_chain_alpha, dim3(1), dim3(1024), 0, st, partials, nph, cs,
-                           chain_alpha());
+        const int np = nph <= kAlphaFold ? nph : 0;
+        if (np == 0)
+            hipLaunchKernelGGL(k_chain_alpha, dim3(1), dim3(1024), 0, st, partials, nph, cs,
+                               chain_alpha());
         if (prec == DMED_FP32)
             hipLaunchKernelGGL(k_chain_update<float>, dim3(g), dim3(kVecBS), 0, st, (float *)w,
-                               (const float *)v, (const float *)vp, n, cs, partials);
+                               (const float *)v, (const float *)vp, n, cs, pu, partials, np, chain_alpha());
         else
             hipLaunchKernelGGL(k_chain_update<double>, dim3(g), dim3(kVecBS), 0, st, (double *)w,
-                               (const double *)v, (const double *)vp, n, cs, partials);
-        hipLaunchKernelGGL(k_chain_beta, dim3(1), dim3(1024), 0, st, partials, (int)g, cs,
-                           chain_beta());
+                               (const double *)v, (const double *)vp, n, cs, pu, partials, np, chain_alpha());
+        hipLaunchKernelGGL(k_chain_beta, dim3(1), dim3(1024), 0, st, pu, (int)g, cs, chain_beta());
         return hipGetLastError() == hipSuccess ? 0 : fail(DMED_EHIP, "chain step launch failed");
     };
     void *vp = bufs[0], *v = bufs[1], *w = bufs[2];
@@ -1062,7 +1082,7 @@ static int chain_run_ws(const dmed_sector *s, const void *v0, int v0prec, int nl
 static size_t chain_nparts(const dmed_sector *s)
 {
     const int nparts = std::max(hxv_nparts(s, DMED_FP64), hxv_nparts(s, DMED_FP32));
-    return (size_t)std::max(nparts, 2 * kVecGrid) + 16;
+    return (size_t)nparts + 2 * kVecGrid + 16;
 }
 
 int chain_run(const dmed_sector *s, const void *v0, int v0prec, int nlanc, int prec,
@@ -1281,7 +1301,7 @@ int plain_gs(const dmed_sector *s, int maxit, double tol, double *eval, dmed_vec
         for (int k = 0; k < 3; ++k)
             if (int rc = exec_buf(ex(), kSlotChainLo + k, n1 * 4, &b32[k])) return rc;
     const int nparts = std::max(hxv_nparts(s, DMED_FP64), hxv_nparts(s, DMED_FP32));
-    if (int rc = ensure_partials(std::max(nparts, 2 * kVecGrid) + 16)) return rc;
+    if (int rc = ensure_partials(nparts + 2 * kVecGrid + 16)) return rc;
     double *psi = nullptr;
     DMED_HIP(hipMalloc(&psi, n1 * 8));
     dmed_vec *out = new dmed_vec{s, DMED_FP64, n, psi};
