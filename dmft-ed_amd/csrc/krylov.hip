@@ -369,6 +369,116 @@ __device__ __forceinline__ double psum_all(const double *__restrict__ p, int n, 
     return s;
 }
 
+// A Lanczos step in two launches, for vectors that fit the caches: H*v leaves y
+// = Hx unscaled, and k_chain_fold does the rest.  It first ends the step before
+// (as k_chain_beta: the norm and <x, x_prev> from that step's partials pp),
+// then alpha from the partials pa of H*v, then the update; every block takes
+// the sums for itself, block 0 stores the results.  What a launch reads of the
+// step before (scalars *cp, partials pp) another one writes (*co, po): two sets
+// taken in turn.  hv is what the next H*v reads: scale 1 and whether the chain
+// has ended.  cp->pad: no partials pending.  A step at D = 853,776: 29.0 -> 24.0 us
+// (FP64), 26.1 -> 21.0 us (FP32); at 203,280: 20.6 -> 16.7 us.
+constexpr int64_t kFoldMaxDim = (int64_t)1 << 22;
+
+// the scalars after a step with ||w||^2 = s, <w, x> = q
+__device__ __forceinline__ void chain_advance(ChainScalars &c, double s, double q)
+{
+    c.b = sqrt(s);
+    c.q = q;
+    c.svp = c.sx;
+    c.sx = 1.0 / c.b;
+    c.step += 1;
+    if (fabs(c.b) < c.thr || c.step >= c.nlanc) c.done = 1;
+}
+
+__global__ void __launch_bounds__(64) k_chain_fold_begin(const ChainScalars *cs, ChainScalars *co,
+                                                         ChainScalars *hv)
+{
+    if (threadIdx.x != 0) return;
+    *co = *cs;
+    co->pad = 1;
+    hv->sx = 1.0;
+    hv->done = cs->done;
+}
+
+__global__ void __launch_bounds__(kVecBS) k_chain_fold_end(const ChainScalars *cp,
+                                                           const double *__restrict__ pp, int g,
+                                                           ChainScalars *cs, double *__restrict__ beta)
+{
+    __shared__ double red[16];
+    ChainScalars c = *cp;
+    const bool adv = !c.pad && !c.done;
+    const double s = psum_all(pp, g, red), q = psum_all(pp + g, g, red);
+    if (threadIdx.x != 0) return;
+    if (adv) {
+        chain_advance(c, s, q);
+        if (c.step < c.nlanc) beta[c.step] = c.b;
+    }
+    c.pad = 0;
+    *cs = c;
+}
+
+template <typename T>
+__global__ void __launch_bounds__(kVecBS) k_chain_fold(
+    T *__restrict__ w, const T *__restrict__ v, const T *__restrict__ vp, int64_t n,
+    const ChainScalars *__restrict__ cp, const double *__restrict__ pp, ChainScalars *__restrict__ co,
+    ChainScalars *__restrict__ hv, double *__restrict__ po, const double *__restrict__ pa, int np,
+    double *__restrict__ alpha, double *__restrict__ beta)
+{
+    constexpr int U = 4;
+    __shared__ double red[16];
+    const bool first = blockIdx.x == 0 && threadIdx.x == 0;
+    ChainScalars c = *cp;
+    if (!c.pad && !c.done) {
+        const double s = psum_all(pp, gridDim.x, red), q = psum_all(pp + gridDim.x, gridDim.x, red);
+        chain_advance(c, s, q);
+        if (first && c.step < c.nlanc) beta[c.step] = c.b;
+    }
+    c.pad = 0;
+    double al = 0.0;
+    if (!c.done) {
+        al = c.sx * (c.sx * psum_any(pa, np, red) - c.b * c.svp * c.q);
+        c.alpha = al;
+    }
+    if (first) {
+        *co = c;
+        hv->sx = 1.0;
+        hv->done = c.done;
+        if (!c.done) alpha[c.step] = al;
+    }
+    if (c.done) return;
+    const double sx = c.sx, ca = al * sx, cb = c.b * c.svp;
+    double s1 = 0.0, s2 = 0.0;
+    const int64_t stride = (int64_t)gridDim.x * blockDim.x;
+    for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += U * stride) {
+        T a[U], b[U], d[U];
+#pragma unroll
+        for (int k = 0; k < U; ++k) {
+            const int64_t e = min(i + k * stride, n - 1);
+            a[k] = w[e];
+            b[k] = v[e];
+            d[k] = vp[e];
+        }
+#pragma unroll
+        for (int k = 0; k < U; ++k) {
+            if (i + k * stride >= n) break;
+            const double vi = (double)b[k];
+            const T wt = (T)(sx * (double)a[k] - cb * (double)d[k] - ca * vi);
+            w[i + k * stride] = wt;
+            const double wi = (double)wt;
+            s1 += wi * wi;
+            s2 += wi * vi;
+        }
+    }
+    s1 = bsum(s1, red);
+    __syncthreads();
+    s2 = bsum(s2, red);
+    if (threadIdx.x == 0) {
+        po[blockIdx.x] = s1;
+        po[gridDim.x + blockIdx.x] = s2;
+    }
+}
+
 // c[r] = sum of the 1 <= g <= kGsGrid partials of row r of P (row stride
 // g), r < nr, into shared c; sixteen rows at a time with all their loads
 // issued before the first add (unconditional, at clamped indices, as in
@@ -916,7 +1026,7 @@ static bool graphs_enabled()
 }
 
 int chain_steps(const dmed_sector *s, void *bufs[3], int prec, int count, double *psi,
-                double *partials, bool allow_graphs = true)
+                double *partials, bool allow_graphs = true, bool two_launch = false)
 {
     hipStream_t st = ex().stream;
     const int64_t n = s->dim;
@@ -927,8 +1037,28 @@ int chain_steps(const dmed_sector *s, void *bufs[3], int prec, int count, double
     const int nph = hxv_nparts(s, prec);
     const unsigned g = vec_grid(n);
     double *pu = partials + nph;        // the update's sums, beside those of H*v
+    // two launches a step: sums and scalars of the two sets in turn
+    const bool fold = two_launch && !psi && n <= kFoldMaxDim && nph <= kAlphaFold;
+    const unsigned gf = std::min<unsigned>(g, kGsGrid);
+    double *fp[2] = {pu, pu + 2 * kGsGrid};
+    ChainScalars *fc = reinterpret_cast<ChainScalars *>(pu + 4 * kGsGrid);   // c[0..1], hv[0..1]
+    int par = 0;                        // set the next step writes
     // the kernels of one step; no memsets, no host synchronisation
     auto one = [&](void *vp, void *v, void *w) -> int {
+        if (fold) {
+            ChainScalars *cp = fc + (par ^ 1), *hp = fc + 2 + (par ^ 1);
+            if (int rc = launch_hxv(s, v, w, prec, kLanczos, hp, partials, nullptr, st)) return rc;
+            if (prec == DMED_FP32)
+                hipLaunchKernelGGL(k_chain_fold<float>, dim3(gf), dim3(kVecBS), 0, st, (float *)w,
+                                   (const float *)v, (const float *)vp, n, cp, fp[par ^ 1], fc + par,
+                                   fc + 2 + par, fp[par], partials, nph, chain_alpha(), chain_beta());
+            else
+                hipLaunchKernelGGL(k_chain_fold<double>, dim3(gf), dim3(kVecBS), 0, st, (double *)w,
+                                   (const double *)v, (const double *)vp, n, cp, fp[par ^ 1], fc + par,
+                                   fc + 2 + par, fp[par], partials, nph, chain_alpha(), chain_beta());
+            par ^= 1;
+            return hipGetLastError() == hipSuccess ? 0 : fail(DMED_EHIP, "chain step launch failed");
+        }
         if (psi) {
             if (prec == DMED_FP32)
                 hipLaunchKernelGGL(k_accum<float>, dim3(g), dim3(kVecBS), 0, st, psi,
@@ -961,7 +1091,11 @@ int chain_steps(const dmed_sector *s, void *bufs[3], int prec, int count, double
         v = w;
         w = t;
     };
+    if (fold) hipLaunchKernelGGL(k_chain_fold_begin, dim3(1), dim3(64), 0, st, cs, fc + 1, fc + 3);
     int k = 0;
+    // steps of a captured window: the buffers (three) and the sets (two) are
+    // back where they started after it
+    const int win = fold ? 6 : 3;
     if (count >= kGraphMinSteps && allow_graphs && graphs_enabled()) {
         // one eager step first (kernel attributes are set outside the capture)
         if (int rc = one(vp, v, w)) return rc;
@@ -972,16 +1106,16 @@ int chain_steps(const dmed_sector *s, void *bufs[3], int prec, int count, double
         // nothing recorded during a capture has run: if the capture fails
         // part-way, the eager loop below resumes from these buffers
         void *const keep[3] = {vp, v, w};
+        const int keep_par = par;
         bool ok = hipStreamBeginCapture(st, hipStreamCaptureModeThreadLocal) == hipSuccess;
         if (ok) {
             int rc = 0;
             const int fail_at = capture_fail_step();
-            for (int q = 0; q < 3 && !rc; ++q) {
+            for (int q = 0; q < win && !rc; ++q) {
                 rc = q == fail_at ? fail(DMED_EHIP, "capture failure forced for a test")
                                   : one(vp, v, w);
                 rotate();
             }
-            // after three rotations the buffers are back where they started
             ok = hipStreamEndCapture(st, &gr) == hipSuccess && rc == 0 && gr != nullptr;
             ok = ok && hipGraphInstantiate(&ge, gr, nullptr, nullptr, 0) == hipSuccess;
         }
@@ -989,16 +1123,17 @@ int chain_steps(const dmed_sector *s, void *bufs[3], int prec, int count, double
             vp = keep[0];
             v = keep[1];
             w = keep[2];
+            par = keep_par;
         }
         bool launched_fail = false;
         if (ok) {
-            const int reps = (count - k) / 3;
+            const int reps = (count - k) / win;
             for (int r = 0; r < reps; ++r)
                 if (hipGraphLaunch(ge, st) != hipSuccess) {
                     launched_fail = true;
                     break;
                 }
-            if (!launched_fail) k += 3 * reps;
+            if (!launched_fail) k += win * reps;
             DMED_HIP(hipStreamSynchronize(st));
         }
         if (ge) hipGraphExecDestroy(ge);
@@ -1017,6 +1152,11 @@ int chain_steps(const dmed_sector *s, void *bufs[3], int prec, int count, double
     for (; k < count; ++k) {
         if (int rc = one(vp, v, w)) return rc;
         rotate();
+    }
+    if (fold) {
+        hipLaunchKernelGGL(k_chain_fold_end, dim3(1), dim3(kVecBS), 0, st, fc + (par ^ 1), fp[par ^ 1],
+                           (int)gf, cs, chain_beta());
+        DMED_HIP(hipGetLastError());
     }
     bufs[0] = vp;
     bufs[1] = v;
@@ -1058,16 +1198,17 @@ static int chain_run_ws(const dmed_sector *s, const void *v0, int v0prec, int nl
     if (int rc = launch_zero(chain_beta(), kChainMax * sizeof(double), st)) return rc;
     if (int rc = chain_init(s, bufs, p0, nlanc, threshold, ws.partials)) return rc;
     if (nhead > 0 && nhead < nlanc) {
-        if (int rc = chain_steps(s, bufs, DMED_FP64, nhead, nullptr, ws.partials, allow_graphs))
+        if (int rc = chain_steps(s, bufs, DMED_FP64, nhead, nullptr, ws.partials, allow_graphs, true))
             return rc;
         // the recurrence needs v and v_prev; w is overwritten by the next step
         void *lo[3] = {ws.b32[0], ws.b32[1], ws.b32[2]};
         if (int rc = launch_scale_copy(lo[0], DMED_FP32, bufs[0], DMED_FP64, n, 1.0, st)) return rc;
         if (int rc = launch_scale_copy(lo[1], DMED_FP32, bufs[1], DMED_FP64, n, 1.0, st)) return rc;
-        if (int rc = chain_steps(s, lo, DMED_FP32, nlanc - nhead, nullptr, ws.partials, allow_graphs))
+        if (int rc = chain_steps(s, lo, DMED_FP32, nlanc - nhead, nullptr, ws.partials, allow_graphs, true))
             return rc;
     } else {
-        if (int rc = chain_steps(s, bufs, p0, nlanc, nullptr, ws.partials, allow_graphs)) return rc;
+        if (int rc = chain_steps(s, bufs, p0, nlanc, nullptr, ws.partials, allow_graphs, true))
+            return rc;
     }
     ChainScalars h;
     DMED_HIP(hipMemcpyAsync(alpha, chain_alpha(), nlanc * sizeof(double), hipMemcpyDeviceToHost, st));
