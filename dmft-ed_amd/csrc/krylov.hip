@@ -167,34 +167,16 @@ template <> struct Vec16<float> { using type = float4; };
 // Each thread takes the elements i = tid + k*stride in increasing order, as a
 // plain grid-stride loop would, with four of them loaded before the first is
 // used; the partial sums (hence beta) do not depend on that grouping.
-// np > 0: the np partials pa of <v, y> are summed here, by every block, instead
-// of by k_chain_alpha (block 0 stores alpha).  Up to kAlphaFold of them that
-// costs less than the launch: a step at D = 853,776 takes 29.0 us, not 29.9; past it the
-// re-reads by all blocks cost more.
-constexpr int kAlphaFold = 4096;
 template <typename T>
 __global__ void __launch_bounds__(kVecBS) k_chain_update(T *__restrict__ w, const T *__restrict__ v,
                                                          const T *__restrict__ vp, int64_t n,
-                                                         ChainScalars *cs,
-                                                         double *__restrict__ partials,
-                                                         const double *__restrict__ pa, int np,
-                                                         double *__restrict__ alpha)
+                                                         const ChainScalars *cs,
+                                                         double *__restrict__ partials)
 {
     constexpr int U = 4;
     __shared__ double red[16];
     if (cs->done) return;
-    const double cb = cs->b * cs->svp;
-    double al;
-    if (np > 0) {
-        al = cs->sx * (psum_any(pa, np, red) - cb * cs->q);      // as k_chain_alpha
-        if (blockIdx.x == 0 && threadIdx.x == 0) {
-            cs->alpha = al;
-            alpha[cs->step] = al;
-        }
-    } else {
-        al = cs->alpha;
-    }
-    const double ca = al * cs->sx;
+    const double ca = cs->alpha * cs->sx, cb = cs->b * cs->svp;
     double s1 = 0.0, s2 = 0.0;
     const int64_t stride = (int64_t)gridDim.x * blockDim.x;
     for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += U * stride) {
@@ -369,7 +351,8 @@ __device__ __forceinline__ double psum_all(const double *__restrict__ p, int n, 
     return s;
 }
 
-// A Lanczos step in two launches, for vectors that fit the caches: H*v leaves y
+// A Lanczos step in two launches, up to kFoldMaxDim states and kFoldMaxParts
+// partials of H*v (every block reads them all): H*v leaves y
 // = Hx unscaled, and k_chain_fold does the rest.  It first ends the step before
 // (as k_chain_beta: the norm and <x, x_prev> from that step's partials pp),
 // then alpha from the partials pa of H*v, then the update; every block takes
@@ -377,8 +360,11 @@ __device__ __forceinline__ double psum_all(const double *__restrict__ p, int n, 
 // step before (scalars *cp, partials pp) another one writes (*co, po): two sets
 // taken in turn.  hv is what the next H*v reads: scale 1 and whether the chain
 // has ended.  cp->pad: no partials pending.  A step at D = 853,776: 29.0 -> 24.0 us
-// (FP64), 26.1 -> 21.0 us (FP32); at 203,280: 20.6 -> 16.7 us.
+// (FP64), 26.1 -> 21.0 us (FP32); at 203,280: 20.6 -> 16.7 us; the ground state at
+// 853,776 states 10.2 -> 9.2 ms.  Past the limit the four launches are as good or
+// better (D = 1.2e7, FP32: 127.1 us, and 137.3 here).
 constexpr int64_t kFoldMaxDim = (int64_t)1 << 22;
+constexpr int kFoldMaxParts = 4096;
 
 // the scalars after a step with ||w||^2 = s, <w, x> = q
 __device__ __forceinline__ void chain_advance(ChainScalars &c, double s, double q)
@@ -1026,7 +1012,7 @@ static bool graphs_enabled()
 }
 
 int chain_steps(const dmed_sector *s, void *bufs[3], int prec, int count, double *psi,
-                double *partials, bool allow_graphs = true, bool two_launch = false)
+                double *partials, bool allow_graphs = true)
 {
     hipStream_t st = ex().stream;
     const int64_t n = s->dim;
@@ -1036,9 +1022,10 @@ int chain_steps(const dmed_sector *s, void *bufs[3], int prec, int count, double
                               chain_aux(), st);
     const int nph = hxv_nparts(s, prec);
     const unsigned g = vec_grid(n);
-    double *pu = partials + nph;        // the update's sums, beside those of H*v
-    // two launches a step: sums and scalars of the two sets in turn
-    const bool fold = two_launch && !psi && n <= kFoldMaxDim && nph <= kAlphaFold;
+    // two launches a step: sums and scalars of the two sets in turn, beside the
+    // sums of H*v
+    const bool fold = n <= kFoldMaxDim && nph <= kFoldMaxParts;
+    double *pu = partials + nph;
     const unsigned gf = std::min<unsigned>(g, kGsGrid);
     double *fp[2] = {pu, pu + 2 * kGsGrid};
     ChainScalars *fc = reinterpret_cast<ChainScalars *>(pu + 4 * kGsGrid);   // c[0..1], hv[0..1]
@@ -1056,6 +1043,14 @@ int chain_steps(const dmed_sector *s, void *bufs[3], int prec, int count, double
                 hipLaunchKernelGGL(k_chain_fold<double>, dim3(gf), dim3(kVecBS), 0, st, (double *)w,
                                    (const double *)v, (const double *)vp, n, cp, fp[par ^ 1], fc + par,
                                    fc + 2 + par, fp[par], partials, nph, chain_alpha(), chain_beta());
+            if (psi) {      // psi += z_k v_k, with the step's scalars just stored
+                if (prec == DMED_FP32)
+                    hipLaunchKernelGGL(k_accum<float>, dim3(g), dim3(kVecBS), 0, st, psi,
+                                       (const float *)v, n, fc + par, chain_aux());
+                else
+                    hipLaunchKernelGGL(k_accum<double>, dim3(g), dim3(kVecBS), 0, st, psi,
+                                       (const double *)v, n, fc + par, chain_aux());
+            }
             par ^= 1;
             return hipGetLastError() == hipSuccess ? 0 : fail(DMED_EHIP, "chain step launch failed");
         }
@@ -1069,17 +1064,16 @@ int chain_steps(const dmed_sector *s, void *bufs[3], int prec, int count, double
         }
         if (int rc = launch_hxv(s, v, w, prec, kLanczos, cs, partials, nullptr, st))
             return rc;
-        const int np = nph <= kAlphaFold ? nph : 0;
-        if (np == 0)
-            hipLaunchKernelGGL(k_chain_alpha, dim3(1), dim3(1024), 0, st, partials, nph, cs,
-                               chain_alpha());
+        hipLaunchKernelGGL(k_chain_alpha, dim3(1), dim3(1024), 0, st, partials, nph, cs,
+                           chain_alpha());
         if (prec == DMED_FP32)
             hipLaunchKernelGGL(k_chain_update<float>, dim3(g), dim3(kVecBS), 0, st, (float *)w,
-                               (const float *)v, (const float *)vp, n, cs, pu, partials, np, chain_alpha());
+                               (const float *)v, (const float *)vp, n, cs, partials);
         else
             hipLaunchKernelGGL(k_chain_update<double>, dim3(g), dim3(kVecBS), 0, st, (double *)w,
-                               (const double *)v, (const double *)vp, n, cs, pu, partials, np, chain_alpha());
-        hipLaunchKernelGGL(k_chain_beta, dim3(1), dim3(1024), 0, st, pu, (int)g, cs, chain_beta());
+                               (const double *)v, (const double *)vp, n, cs, partials);
+        hipLaunchKernelGGL(k_chain_beta, dim3(1), dim3(1024), 0, st, partials, (int)g, cs,
+                           chain_beta());
         return hipGetLastError() == hipSuccess ? 0 : fail(DMED_EHIP, "chain step launch failed");
     };
     void *vp = bufs[0], *v = bufs[1], *w = bufs[2];
@@ -1198,17 +1192,16 @@ static int chain_run_ws(const dmed_sector *s, const void *v0, int v0prec, int nl
     if (int rc = launch_zero(chain_beta(), kChainMax * sizeof(double), st)) return rc;
     if (int rc = chain_init(s, bufs, p0, nlanc, threshold, ws.partials)) return rc;
     if (nhead > 0 && nhead < nlanc) {
-        if (int rc = chain_steps(s, bufs, DMED_FP64, nhead, nullptr, ws.partials, allow_graphs, true))
+        if (int rc = chain_steps(s, bufs, DMED_FP64, nhead, nullptr, ws.partials, allow_graphs))
             return rc;
         // the recurrence needs v and v_prev; w is overwritten by the next step
         void *lo[3] = {ws.b32[0], ws.b32[1], ws.b32[2]};
         if (int rc = launch_scale_copy(lo[0], DMED_FP32, bufs[0], DMED_FP64, n, 1.0, st)) return rc;
         if (int rc = launch_scale_copy(lo[1], DMED_FP32, bufs[1], DMED_FP64, n, 1.0, st)) return rc;
-        if (int rc = chain_steps(s, lo, DMED_FP32, nlanc - nhead, nullptr, ws.partials, allow_graphs, true))
+        if (int rc = chain_steps(s, lo, DMED_FP32, nlanc - nhead, nullptr, ws.partials, allow_graphs))
             return rc;
     } else {
-        if (int rc = chain_steps(s, bufs, p0, nlanc, nullptr, ws.partials, allow_graphs, true))
-            return rc;
+        if (int rc = chain_steps(s, bufs, p0, nlanc, nullptr, ws.partials, allow_graphs)) return rc;
     }
     ChainScalars h;
     DMED_HIP(hipMemcpyAsync(alpha, chain_alpha(), nlanc * sizeof(double), hipMemcpyDeviceToHost, st));
