@@ -237,7 +237,7 @@ static_assert(kColHeadBytes % 256 == 0, "the column starts on a DMA boundary");
 // opposite occupations), the same for all its rows.  Most pairs take a column
 // nowhere and are skipped by the whole workgroup; of the rest the rows whose
 // own hop exists gather from the other column.  Three orbitals, D = 853,776,
-// FP64: tile kernel 34.8 us, here 13 us (without the pairs 7.8 us); a Lanczos
+// FP64: tile kernel 34.8 us, here 14 us (without the pairs 9 us); a Lanczos
 // step at D = 4.1e7: 2.10 -> 0.96 ms.
 struct ColPairs {
     const int32_t *ju, *jd;

@@ -651,8 +651,8 @@ __global__ void __launch_bounds__(kVecBS) k_trl_local(double *__restrict__ w,
 // them.  The basis is read twice for two steps instead of four times (or
 // more, with the gated second passes, which a remainder of rounding size
 // never needs), and the two steps take seven launches instead of fourteen.
-// Bound by those reads of the basis.  Lowest pair of an 853,776-state sector
-// to 1e-12 (20 basis vectors): 54 -> 41 ms.
+// Bound by those reads of the basis.  Four lowest pairs of an 853,776-state
+// sector to 1e-12 (20 basis vectors): 54 -> 41 ms.
 //
 // With r the remainder of w1, |r| ~ eps |H|: alpha is off by 2 <v_j, r> and the
 // part s H r of w2 lies in the span that the pass takes off, so alpha, beta and
