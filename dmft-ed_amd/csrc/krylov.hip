@@ -715,6 +715,15 @@ __global__ void __launch_bounds__(kVecBS) k_trl_second(double *__restrict__ w2,
     }
 }
 
+// Every block of k_proj_axpy2 sums all partials of k_proj_dot2 for itself.  Up
+// to kPairMidDim states that costs as much as the basis: 128 blocks of two rows
+// leave a quarter of the partials of 512 blocks of eight (four lowest pairs at
+// 853,776 states 42.4 -> 40.7 ms, at 63,504 states 16.6 -> 15.6 ms); longer
+// vectors need the blocks and the shared reads of w1, w2 (2,944,656 states:
+// 112.0 ms, and 115.9 with 128 by two).
+constexpr int64_t kPairMidDim = (int64_t)1 << 20;
+static unsigned pair_grid(int64_t n) { return n <= kPairMidDim ? 128 : kGsGrid; }
+
 // Partials of the projections of w1 and w2 on the rows Y_0..Y_{ny-1},
 // V_0..V_{nv-1}: P[(2r)*gridDim.x + block] and P[(2r+1)*gridDim.x + block]; and
 // of <w1, w2> in row 2*(ny+nv).  rpb rows a block, as in k_proj_dot.
@@ -768,18 +777,18 @@ __global__ void __launch_bounds__(kVecBS) k_proj_dot2(
 
 // v = s w1 - sum_r row_r c1_r (in place of w1) and w2 -= sum_r row_r c2_r +
 // <v', w2> v' with v' = s w1, s = 1/*beta and the coefficients from the
-// partials of k_proj_dot2 (c1 scaled by s); block partials of the new
+// gp partials a row of k_proj_dot2 (c1 scaled by s); block partials of the new
 // ||w2||^2 in Pn.
 __global__ void __launch_bounds__(kVecBS) k_proj_axpy2(
     const double *__restrict__ Y, int ny, const double *__restrict__ V, int nv,
-    double *__restrict__ w1, double *__restrict__ w2, int64_t n, const double *__restrict__ P,
+    double *__restrict__ w1, double *__restrict__ w2, int64_t n, const double *__restrict__ P, int gp,
     const double *__restrict__ beta, double *__restrict__ Pn)
 {
     __shared__ double red[16];
     __shared__ double red16[16 * (kVecBS / 64)];
     __shared__ double c[2 * kGsMaxRows + 1];
     const int nr = ny + nv;
-    rowsums(P, 2 * nr + 1, gridDim.x, c, red16);
+    rowsums(P, 2 * nr + 1, gp, c, red16);
     const double be = *beta, sc = be > 0.0 ? 1.0 / be : 0.0;
     const double cab = sc * c[2 * nr];
     double s2 = 0.0;
@@ -1652,11 +1661,12 @@ int trl_run(const dmed_sector *s, int neig, int m, int maxit, double tol, const 
         if (int rc = launch_hxv(s, w1, w, DMED_FP64, kLanczos, tcs, Pa, nullptr, st)) return rc;
         hipLaunchKernelGGL(k_trl_second, dim3(g), dim3(kVecBS), 0, st, w, w1, vj, n, Pa, nph, Pw, cj,
                            cj1, j, m);
-        const int rows = nl + j + 1, rpb = proj_rpb(n);
-        hipLaunchKernelGGL(k_proj_dot2, dim3(g, proj_groups(rows, rpb)), dim3(kVecBS), 0, st, Y, nl, V,
+        const unsigned gp = std::min(g, pair_grid(n));
+        const int rows = nl + j + 1, rpb = std::min(proj_rpb(n), n <= kPairMidDim ? 2 : kProjRows);
+        hipLaunchKernelGGL(k_proj_dot2, dim3(gp, proj_groups(rows, rpb)), dim3(kVecBS), 0, st, Y, nl, V,
                            j + 1, w1, w, n, P1, rpb);
         hipLaunchKernelGGL(k_proj_axpy2, dim3(g), dim3(kVecBS), 0, st, Y, nl, V, j + 1, w1, w, n, P1,
-                           cj + m + 1, Pn2);
+                           (int)gp, cj + m + 1, Pn2);
         hipLaunchKernelGGL(k_normalize, dim3(g), dim3(kVecBS), 0, st, w1 + n, w, n, Pn2, Pn2, Pn2, 1,
                            cj1 + m + 1);
         DMED_HIP(hipGetLastError());
