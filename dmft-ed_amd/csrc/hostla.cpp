@@ -24,6 +24,7 @@ static double hyp(double a, double b)
     // the pythag of ED_GREENS_FUNCTIONS.f90:513-539)
     double p = std::max(std::fabs(a), std::fabs(b));
     if (std::isnan(a) || std::isnan(b)) return NAN;
+    if (std::isinf(p)) return p;        // the ratio below would be NaN and never settle
     if (p != 0.0) {
         double r = std::min(std::fabs(a), std::fabs(b)) / p;
         r = r * r;
