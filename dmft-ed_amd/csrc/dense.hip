@@ -63,6 +63,21 @@ __device__ __forceinline__ double dsum(double v, double *red)
     return s;
 }
 
+// Place of level i among d[0..n): ascending, equal levels by index, and levels
+// that are not a number after all others, by index.  A total order, so that
+// the places of all levels are 0..n-1 each once, whatever d holds.
+__host__ __device__ inline int level_place(const double *d, int n, int i)
+{
+    const double x = d[i];
+    int p = 0;
+    for (int j = 0; j < n; ++j) {
+        const double y = d[j];
+        const bool before = x == x ? y < x || (y == x && j < i) : y == y || j < i;
+        p += before ? 1 : 0;
+    }
+    return p;
+}
+
 // H of the sector into A (column-major), a row per lane: the terms of
 // k_hxv's row sum
 __device__ void build_h(const DenseTask &t)
@@ -283,14 +298,12 @@ __global__ void __launch_bounds__(kDenseBlock) k_dense_eigh(const DenseTask *__r
         __syncthreads();
         if (!pub[it & 1][2]) break;
     }
-    // ascending selection of the wanted eigenvalues: rank by counting, ties
-    // by index
+    // ascending selection of the wanted eigenvalues; a level that is not finite
+    // (a model with NaN or infinity) is reported like one that did not converge
     int *order = reinterpret_cast<int *>(v);
     for (int i = tid; i < n; i += kDenseBlock) {
-        const double x = d[i];
-        int rk = 0;
-        for (int j = 0; j < n; ++j) rk += d[j] < x || (d[j] == x && j < i);
-        order[rk] = i;
+        order[level_place(d, n, i)] = i;
+        if (!isfinite(d[i])) bad = 1;
     }
     __syncthreads();
     // back-transformation, a wave per eigenvector: y -= v_k (v_k . y)
@@ -314,6 +327,12 @@ __global__ void __launch_bounds__(kDenseBlock) k_dense_eigh(const DenseTask *__r
 }  // namespace
 
 bool dense_takes(int64_t n) { return n >= 1 && n <= kDenseMaxDim; }
+
+// order[q] = index of the q-th level, by the rule of k_dense_eigh
+void dense_order(int n, const double *d, int *order)
+{
+    for (int i = 0; i < n; ++i) order[level_place(d, n, i)] = i;
+}
 
 // Launch the items on e's stream (asynchronous); dense_finish waits.
 int dense_launch(DenseBatch &b, Exec &e)

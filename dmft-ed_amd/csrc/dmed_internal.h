@@ -352,6 +352,7 @@ struct DenseBatch {
     size_t nev = 0;
 };
 bool dense_takes(int64_t n);
+void dense_order(int n, const double *d, int *order);
 int dense_launch(DenseBatch &b, Exec &e);
 int dense_finish(DenseBatch &b);
 
