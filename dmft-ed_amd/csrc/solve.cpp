@@ -359,6 +359,7 @@ extern "C" int dmed_solve(const dmed_solve_params *p, dmed_solve_out *out)
             neigen[is] = out->neigen_sector && out->neigen_sector[is] > 0
                              ? out->neigen_sector[is]
                              : (int)std::min<int64_t>(dim, nst_sector);
+            if (neigen[is] < 1) return fail(DMED_EINVAL, "neig out of range");
         }
 
     const double t0 = now();
