@@ -63,7 +63,7 @@ void exec_destroy(Exec &e)
     e = Exec();
 }
 
-int exec_buf(Exec &e, int slot, size_t bytes, void **p)
+int exec_try(Exec &e, int slot, size_t bytes, void **p)
 {
     if (slot < 0 || slot >= kExecSlots) return fail(DMED_EINVAL, "bad buffer slot");
     bytes = std::max<size_t>(bytes, 256);
@@ -74,11 +74,23 @@ int exec_buf(Exec &e, int slot, size_t bytes, void **p)
         }
         e.buf[slot] = nullptr;
         e.buf_cap[slot] = 0;
-        DMED_HIP(hipMalloc(&e.buf[slot], bytes));
+        const hipError_t err = hipMalloc(&e.buf[slot], bytes);
+        if (err == hipErrorOutOfMemory) {
+            (void)hipGetLastError();    // not for the next launch to find
+            e.buf[slot] = nullptr;
+            return DMED_ENOMEM;
+        }
+        DMED_HIP(err);
         e.buf_cap[slot] = bytes;
     }
     *p = e.buf[slot];
     return 0;
+}
+
+int exec_buf(Exec &e, int slot, size_t bytes, void **p)
+{
+    const int rc = exec_try(e, slot, bytes, p);
+    return rc == DMED_ENOMEM ? fail(DMED_EHIP, "hipMalloc of a work buffer: out of memory") : rc;
 }
 
 // Host-to-device copy on the calling thread's stream, finished on return.

@@ -335,6 +335,7 @@ void dense_order(int n, const double *d, int *order)
 }
 
 // Launch the items on e's stream (asynchronous); dense_finish waits.
+// DMED_ENOMEM: no room for the work space, nothing was launched.
 int dense_launch(DenseBatch &b, Exec &e)
 {
     b.exec = &e;
@@ -357,7 +358,7 @@ int dense_launch(DenseBatch &b, Exec &e)
         off += up(2 * n * n * 8) + up((size_t)b.items[k].neig * n * 8);
     }
     unsigned char *d = nullptr;
-    if (int rc = exec_buf(e, kSlotDense, off, (void **)&d)) return rc;
+    if (int rc = exec_try(e, kSlotDense, off, (void **)&d)) return rc;
     b.tasks.resize(nt * sizeof(DenseTask));
     DenseTask *h = reinterpret_cast<DenseTask *>(b.tasks.data());
     double *dev = reinterpret_cast<double *>(d + ores);

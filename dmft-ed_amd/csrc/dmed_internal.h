@@ -156,6 +156,9 @@ void exec_pool_clear();                 // destroys the idle worker contexts (so
 Exec &ex();                             // context of the calling thread
 void bind_exec(Exec *e);                // nullptr: back to the default context
 int exec_buf(Exec &e, int slot, size_t bytes, void **p);
+// the same for a caller with another way: DMED_ENOMEM, without a message and
+// with HIP's error cleared, where device memory is short
+int exec_try(Exec &e, int slot, size_t bytes, void **p);
 
 struct Context {
     bool initialized = false;
@@ -367,6 +370,7 @@ int tql2_first_row(int n, double *d, double *e, double *z1);
 void gf_add_poles(double peso, double ei, const double *lam, const double *w2, int n,
                   int isign, const double *wm, int lmats, const double *wr, int lreal,
                   double eps, double *gm, double *gr);
+bool host_may_take(int rc);             // of a device sum (gf.hip)
 // One chain of a Green's function: weight pr + i pi on
 // <e1| (z - isign*(T - ei))^-1 |e1>, T of alpha[0..n), beta[1..n).
 struct GfTerm {

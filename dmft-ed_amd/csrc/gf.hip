@@ -116,7 +116,7 @@ int gf_sum_device(const std::vector<GfTerm> &terms, const double *wm, int lm, co
         }
     }
     unsigned char *d = nullptr;
-    if (int rc = exec_buf(ex(), kSlotGf, total, (void **)&d)) return rc;
+    if (int rc = exec_try(ex(), kSlotGf, total, (void **)&d)) return rc;
     DMED_HIP(hipMemcpyAsync(d, h.data(), nup, hipMemcpyHostToDevice, st));
     const CfChain *dc = reinterpret_cast<const CfChain *>(d + ohdr);
     double2 *dout = reinterpret_cast<double2 *>(d + oout);
@@ -368,7 +368,7 @@ int chi_sum_device(const std::vector<ChiTerm> &terms, int ntarget, double beta, 
     std::memcpy(h.data() + otoff, toff.data(), toff.size() * 4);
     std::memcpy(h.data() + oab, ab.data(), ab.size() * 8);
     unsigned char *d = nullptr;
-    if (int rc = exec_buf(ex(), kSlotGf, total, (void **)&d)) return rc;
+    if (int rc = exec_try(ex(), kSlotGf, total, (void **)&d)) return rc;
     DMED_HIP(hipMemcpyAsync(d, h.data(), nup, hipMemcpyHostToDevice, st));
     const ChiDev *dt = reinterpret_cast<const ChiDev *>(d + odev);
     double2 *dpole = reinterpret_cast<double2 *>(d + opole);
@@ -428,6 +428,11 @@ int chi_sum_host(const std::vector<ChiTerm> &terms, double beta, const ChiGrid &
 
 }  // namespace
 
+// Whether the host form takes over after a device sum returned rc: where its
+// buffer could not be had or its pole iteration did not converge.  A HIP error
+// goes to the caller.
+bool host_may_take(int rc) { return rc == DMED_ENOMEM || rc == DMED_ENOCONV; }
+
 // g[0..lm) on the Matsubara axis, g[lm..lm+lr) on the real axis, overwritten
 // with the sum over the terms.  The continued fraction needs every point off
 // the real axis (1e-100: its square is still a normal number) and finite
@@ -448,7 +453,10 @@ int gf_sum(const std::vector<GfTerm> &terms, const double *wm, int lm, const dou
     ok = ok && nmax >= kCfMin && (lr == 0 || (std::fabs(eps) > 1e-100 && std::fabs(eps) < 1e100));
     for (int i = 0; i < lm && ok; ++i) ok = std::fabs(wm[i]) > 1e-100 && std::fabs(wm[i]) < 1e100;
     for (int i = 0; i < lr && ok; ++i) ok = std::fabs(wr[i]) < 1e100;
-    if (ok && gf_sum_device(terms, wm, lm, wr, lr, eps, g) == 0) return 0;
+    if (ok) {
+        const int rc = gf_sum_device(terms, wm, lm, wr, lr, eps, g);
+        if (!host_may_take(rc)) return rc;
+    }
     return gf_sum_host(terms, wm, lm, wr, lr, eps, g);
 }
 
@@ -474,7 +482,10 @@ int chi_sum(std::vector<ChiTerm> terms, int ntarget, double beta, const ChiGrid 
             ok = std::fabs(t.alpha[i]) < 1e100 && (i == 0 || std::fabs(t.beta[i]) < 1e100);
     }
     ok = ok && nmax >= kChiMin && nmax <= kChiMaxSteps && nsum < ((size_t)1 << 24);     // 64 B of work space a pole
-    if (ok && chi_sum_device(terms, ntarget, beta, g, out) == 0) return 0;
+    if (ok) {
+        const int rc = chi_sum_device(terms, ntarget, beta, g, out);
+        if (!host_may_take(rc)) return rc;
+    }
     std::fill(out, out + 2 * (size_t)ntarget * (g.nv + g.nt + g.lr), 0.0);
     return chi_sum_host(terms, beta, g, out);
 }

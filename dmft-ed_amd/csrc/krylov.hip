@@ -1925,7 +1925,9 @@ int eigh_sector_ex(const dmed_sector *s, int neig, int ncv, int maxit, double to
             it.lowest = lowest_multiplet;
             it.degen = degen;
             it.want_vecs = evecs != nullptr;
-            if (dense_launch(b, ex()) == 0 && dense_finish(b) == 0 && it.rc == 0) {
+            int rc = dense_launch(b, ex());
+            if (!rc) rc = dense_finish(b);
+            if (!rc && it.rc == 0) {
                 *nout = it.nout;
                 for (int q = 0; q < it.nout; ++q) {
                     evals[q] = it.evals[q];
@@ -1935,6 +1937,8 @@ int eigh_sector_ex(const dmed_sector *s, int neig, int ncv, int maxit, double to
                 return 0;
             }
             for (dmed_vec *v : it.vecs) dmed_vec_free(v);
+            if (rc && rc != DMED_ENOMEM) return rc;
+            // no room or no convergence: the host
         }
         if (!lowest_multiplet) {
             *nout = neig;

@@ -476,8 +476,12 @@ extern "C" int dmed_solve(const dmed_solve_params *p, dmed_solve_out *out)
         std::vector<Exec *> dex;
         int drc = 0;
         if (!db.items.empty()) {
-            drc = pool_acquire(1, dex);
-            if (!drc) drc = dense_launch(db, *dex[0]);
+            if (pool_acquire(1, dex)) {
+                (void)hipGetLastError();
+                drc = DMED_ENOMEM;
+            } else {
+                drc = dense_launch(db, *dex[0]);
+            }
         }
         hipStream_t qs = nullptr;
         const double tq0 = now();
@@ -496,8 +500,12 @@ extern "C" int dmed_solve(const dmed_solve_params *p, dmed_solve_out *out)
         for (size_t k = 0; k < dsec.size() && !rc; ++k) {
             DenseItem &it = db.items[k];
             SectorRes &r = sres[dsec[k]];
+            if (drc && drc != DMED_ENOMEM) {
+                rc = drc;
+                break;
+            }
             if (drc || it.rc) {
-                // the batch could not run or did not converge: one by one
+                // the batch had no room or did not converge: one by one
                 for (dmed_vec *v : it.vecs) dmed_vec_free(v);
                 solve_sector(dsec[k]);
                 continue;
