@@ -8,6 +8,7 @@
 #include <cmath>
 #include <complex>
 #include <cstdio>
+#include <cstdlib>
 #include <cstring>
 #include <map>
 #include <memory>
@@ -66,6 +67,9 @@ void exec_destroy(Exec &e)
 int exec_try(Exec &e, int slot, size_t bytes, void **p)
 {
     if (slot < 0 || slot >= kExecSlots) return fail(DMED_EINVAL, "bad buffer slot");
+    // DMED_TEST_NO_MEMORY=slot: no room for that buffer
+    if (const char *t = std::getenv("DMED_TEST_NO_MEMORY"))
+        if (std::atoi(t) == slot) return DMED_ENOMEM;
     bytes = std::max<size_t>(bytes, 256);
     if (bytes > e.buf_cap[slot]) {
         if (e.buf[slot]) {

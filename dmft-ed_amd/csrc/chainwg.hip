@@ -391,7 +391,7 @@ int chain_batch_run(std::vector<ChainBatchItem> &items, double threshold)
     for (auto &it : items) ncoef += 2 * (size_t)it.nlanc;
     const size_t nargs = (items.size() * sizeof(WgArgs<double>) + 255) / 256 * 256;
     char *buf = nullptr;
-    if (int rc = exec_buf(ex(), kSlotChainBatch, nargs + ncoef * 8, (void **)&buf)) return rc;
+    if (int rc = exec_try(ex(), kSlotChainBatch, nargs + ncoef * 8, (void **)&buf)) return rc;
     double *coef = reinterpret_cast<double *>(buf + nargs);
     std::vector<WgArgs<double>> args;
     for (int k : order) {

@@ -280,6 +280,7 @@ struct ChainBatchItem {
     double *alpha, *beta;
 };
 bool chain_batch_takes(const dmed_sector *s, int nlanc);
+// DMED_ENOMEM: no room for the descriptors, some chains may not have run
 int chain_batch_run(std::vector<ChainBatchItem> &items, double threshold);
 int eigh_sector(const dmed_sector *s, int neig, int ncv, int maxit, double tol,
                 int dense_threshold, double *evals, dmed_vec **evecs, double *resid);

@@ -249,7 +249,10 @@ struct ChainPhase {
             refs[t].off = total;
             total += bytes;
         }
-        return total ? exec_buf(ex(), kSlotBatchVec, total, (void **)&slab) : 0;
+        const int rc = total ? exec_try(ex(), kSlotBatchVec, total, (void **)&slab) : 0;
+        if (rc == DMED_ENOMEM)              // no slab: every chain by its task
+            for (Ref &r : refs) r.off = SIZE_MAX;
+        return rc == DMED_ENOMEM ? 0 : rc;
     }
     // where task t puts its start vector, null: in a buffer of its own
     void *place(int t) { return refs[t].off == SIZE_MAX ? nullptr : slab + refs[t].off; }
@@ -259,7 +262,15 @@ struct ChainPhase {
         for (Ref &r : refs)
             if (r.ready)
                 items.push_back({r.s, slab + r.off, (int)r.al->size(), r.al->data(), r.bl->data()});
-        return chain_batch_run(items, 1e-13);
+        int rc = chain_batch_run(items, 1e-13);
+        if (rc != DMED_ENOMEM) return rc;
+        rc = 0;                             // no room for the batch: one by one
+        for (size_t k = 0; k < items.size() && !rc; ++k) {
+            const ChainBatchItem &it = items[k];
+            rc = chain_run(it.s, it.v, DMED_FP64, it.nlanc, DMED_FP64, 1e-13, it.alpha, it.beta,
+                           nullptr, kMixedHead);
+        }
+        return rc;
     }
 };
 

@@ -39,3 +39,27 @@ def test_memory_that_cannot_be_had_leaves_nothing_behind():
     assert np.array_equal(s.hxv(x), want)           # the launch check sees no old error
     rc, p = _try(17, 1 << 12)
     assert rc == 0 and p
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("slot", [11, 15, 16, 17])
+def test_solve_without_room_for_a_buffer(slot, monkeypatch):
+    """The solve's answers when one of its optional buffers cannot be had: the
+    sums of G and chi (11), the dense sectors (15), the slab of start vectors
+    (16) and the descriptors (17) of the chain batch."""
+    dmed.init(0)
+    rng = np.random.default_rng(4)
+    bath = np.concatenate([rng.uniform(-1, 1, 5), rng.uniform(0.2, 0.5, 5)])
+    ns = dmed.set_model(1, 5, 1, bath, np.zeros(1), [2.0])
+    p = dmed.default_params(beta=20.0, lmats=64, lreal=10, eps=0.3, batched=1, chi_spin=1, chi_dens=1,
+                            lanc_nstates_sector=4, lanc_nstates_total=20)
+    want = dmed.solve(1, 1, ns, p)
+    monkeypatch.setenv("DMED_TEST_NO_MEMORY", str(slot))
+    print(f"[no memory] slot {slot}", flush=True)
+    got = dmed.solve(1, 1, ns, p)
+    # the same levels and chains to the solver's tolerance of 1e-12, in sums of
+    # condition beta (chi) and 1/min |z| (G); orders of magnitude beyond it
+    assert got["nstates"] == want["nstates"] and abs(got["egs"] - want["egs"]) < 1e-11
+    for k, v in want.items():
+        if isinstance(v, np.ndarray) and v.dtype.kind in "fc":
+            assert np.abs(got[k] - v).max() <= 1e-8 * max(1.0, np.abs(v).max()), k
