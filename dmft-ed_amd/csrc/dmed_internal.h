@@ -335,7 +335,8 @@ int queue_finish(SectorQueue &q);
 
 // ------------------------------------------------ dense sectors (dense.hip)
 // Sectors diagonalised in full, one workgroup each, in one launch.  The
-// sectors must outlive dense_finish, which waits and fills the items.
+// sectors must outlive dense_finish, which waits and fills the items.  An
+// eigenvector left in `vecs` is freed with its item.
 constexpr int64_t kDenseMaxDim = 1024;
 struct DenseItem {
     const dmed_sector *s = nullptr;
@@ -347,6 +348,13 @@ struct DenseItem {
     std::vector<dmed_vec *> vecs;           // out: nout vectors
     int nout = 0, rc = 0;                   // out: rc 0 or DMED_ENOCONV
     const double *dvecs = nullptr;
+    DenseItem() = default;
+    DenseItem(DenseItem &&) = default;
+    DenseItem(const DenseItem &) = delete;
+    ~DenseItem()
+    {
+        for (dmed_vec *v : vecs) dmed_vec_free(v);
+    }
 };
 struct DenseBatch {
     std::vector<DenseItem> items;

@@ -1934,9 +1934,9 @@ int eigh_sector_ex(const dmed_sector *s, int neig, int ncv, int maxit, double to
                     if (resid) resid[q] = 0.0;
                     if (evecs) evecs[q] = it.vecs[q];
                 }
+                it.vecs.clear();
                 return 0;
             }
-            for (dmed_vec *v : it.vecs) dmed_vec_free(v);
             if (rc && rc != DMED_ENOMEM) return rc;
             // no room or no convergence: the host
         }

@@ -517,18 +517,24 @@ extern "C" int dmed_solve(const dmed_solve_params *p, dmed_solve_out *out)
             }
             if (drc || it.rc) {
                 // the batch had no room or did not converge: one by one
-                for (dmed_vec *v : it.vecs) dmed_vec_free(v);
                 solve_sector(dsec[k]);
                 continue;
             }
             r.nout = it.nout;
             r.ev = it.evals;
-            r.vecs = it.vecs;
+            r.vecs = std::move(it.vecs);
+            it.vecs.clear();
         }
         const int frc = queue_finish(q);
         if (!qrc) qrc = frc;
         if (qs) hipStreamDestroy(qs);
-        if (rc) return rc;
+        if (rc) {
+            for (QueueItem &it : q.items)
+                for (dmed_vec *v : it.vecs) dmed_vec_free(v);
+            for (SectorRes &r : sres)
+                for (dmed_vec *v : r.vecs) dmed_vec_free(v);
+            return rc;
+        }
         if (p->verbose > 1 && !q.items.empty())
             std::fprintf(stderr, "sector queue: %d sectors, kernel %.3f ms; %.3f ms with the "
                                  "workers\n", (int)q.items.size(), q.kernel_ms, 1e3 * (now() - tq0));
