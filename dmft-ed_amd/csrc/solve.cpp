@@ -125,17 +125,24 @@ inline size_t gidx(int s1, int s2, int a, int b, int l, int nspin, int norb)
 // distinct ones; at most kPoolKeep idle contexts are kept, and the rest are
 // destroyed on release.  exec_pool_clear (dmed_finalize) destroys them all.
 constexpr int kPoolKeep = 16;
-// work space of the dense sectors of one launch; sectors past it are solved
-// one by one
+// work space of the dense sectors of one launch (H, Z and the eigenvectors);
+// sectors past it are solved one by one
 constexpr size_t kDenseBatchBytes = (size_t)256 << 20;
 std::mutex g_pool_mu;
 std::vector<Exec *> g_pool;
 
-int pool_acquire(int nw, std::vector<Exec *> &out)
+// slot >= 0: idle contexts with the largest buffer of that slot first, so that
+// large ones gather in as few contexts as are in use at once
+int pool_acquire(int nw, std::vector<Exec *> &out, int slot = -1)
 {
     std::lock_guard<std::mutex> lk(g_pool_mu);
     while ((int)out.size() < nw) {
         if (!g_pool.empty()) {
+            if (slot >= 0)
+                std::iter_swap(g_pool.end() - 1,
+                               std::max_element(g_pool.begin(), g_pool.end(), [&](Exec *a, Exec *b) {
+                                   return a->buf_cap[slot] < b->buf_cap[slot];
+                               }));
             out.push_back(g_pool.back());
             g_pool.pop_back();
             continue;
@@ -458,9 +465,10 @@ extern "C" int dmed_solve(const dmed_solve_params *p, dmed_solve_out *out)
             const int ne = (int)std::min<int64_t>(dim, neigen[is]);
             const int nblock = (int)std::min<int64_t>(dim, p->lanc_ncv_factor * ne + p->lanc_ncv_add);
             const int ncv = std::max(nblock, 2 * ne + 10);
+            const size_t db_bytes = 8 * (size_t)dim * (2 * (size_t)dim + ne);
             if ((dim <= p->lanc_dim_threshold || ne == dim) && dense_takes(dim) &&
-                dense_bytes + 16 * (size_t)dim * dim <= kDenseBatchBytes) {
-                dense_bytes += 16 * (size_t)dim * dim;
+                dense_bytes + db_bytes <= kDenseBatchBytes) {
+                dense_bytes += db_bytes;
                 DenseItem it;
                 it.s = secs[is];
                 it.neig = ne;
@@ -487,7 +495,7 @@ extern "C" int dmed_solve(const dmed_solve_params *p, dmed_solve_out *out)
         std::vector<Exec *> dex;
         int drc = 0;
         if (!db.items.empty()) {
-            if (pool_acquire(1, dex)) {
+            if (pool_acquire(1, dex, kSlotDense)) {
                 (void)hipGetLastError();
                 drc = DMED_ENOMEM;
             } else {
