@@ -662,16 +662,18 @@ static ColFit col_fit(const dmed_sector *s, int prec, int bs)
 // The column kernel's Lanczos-mode partial sums are one per column, so a
 // tuned shape changes neither y nor alpha/beta; the tile kernel keeps the
 // fixed rule in Lanczos mode (its partial sums follow the grid).
-// DMED_TUNE_FILE=path loads earlier choices on first use and appends new ones.
+// DMED_TUNE_FILE=path loads earlier choices on first use and appends new ones;
+// a line's fifth number is 2^Norb, negative for a sector with spin exchange and
+// pair hopping, whose kernels are others.
 struct TuneChoice {
     int cb = 0, bs = 0;      // tile kernel (0: fixed rule)
     int cbs = 0, wgs = 0;    // column kernel lanes and workgroups per CU (0: fixed rule)
 };
-using TuneKey = std::tuple<int64_t, int64_t, int, int, int, int>;
+using TuneKey = std::tuple<int64_t, int64_t, int, int, int, int>;   // nimp < 0: jterms
 
 static TuneKey tune_key(const dmed_sector *s, int prec)
 {
-    return TuneKey{s->up->dim, s->dw->dim, s->up->nhop, s->dw->nhop, s->nimp,
+    return TuneKey{s->up->dim, s->dw->dim, s->up->nhop, s->dw->nhop, s->jterms ? -s->nimp : s->nimp,
                    prec == DMED_FP32 ? DMED_FP32 : DMED_FP64};
 }
 
