@@ -687,10 +687,18 @@ extern "C" int dmed_gf_add_chain(double peso_bz, double ei, const double *alpha,
 {
     if (nlanc <= 0) return 0;
     const int lm = std::max(lmats, 0), lr = std::max(lreal, 0);
+    const std::vector<GfTerm> term{GfTerm{alpha, beta, nlanc, isign, ei, peso_bz, 0.0}};
+    if (!gf_on_device(term, wm, lm, wr, lr, eps)) {
+        std::vector<double> d(alpha, alpha + nlanc), e(nlanc, 0.0), z(nlanc);
+        for (int i = 1; i < nlanc; ++i) e[i] = beta[i];
+        if (tql2_first_row(nlanc, d.data(), e.data(), z.data()))
+            return fail(DMED_ENOCONV, "tql2 did not converge");
+        for (auto &x : z) x = x * x;
+        gf_add_poles(peso_bz, ei, d.data(), z.data(), nlanc, isign, wm, lm, wr, lr, eps, gmats, greal);
+        return 0;
+    }
     std::vector<double> g(2 * ((size_t)lm + lr));
-    if (int rc = gf_sum({GfTerm{alpha, beta, nlanc, isign, ei, peso_bz, 0.0}}, wm, lm, wr, lr, eps,
-                        g.data()))
-        return rc;
+    if (int rc = gf_sum(term, wm, lm, wr, lr, eps, g.data())) return rc;
     for (size_t i = 0; i < 2 * (size_t)lm; ++i) gmats[i] += g[i];
     for (size_t i = 0; i < 2 * (size_t)lr; ++i) greal[i] += g[2 * (size_t)lm + i];
     return 0;
@@ -922,12 +930,23 @@ extern "C" int dmed_chi_add_chain(double peso_f, double peso_bz, double ei, cons
         (lreal > 0 && (!wr || !chi_w)))
         return fail(DMED_EINVAL, "null argument");
     const ChiGrid g{vm, tau, wr, std::max(nv, 0), std::max(ntau, 0), std::max(lreal, 0), eps};
-    std::vector<double> o(2 * ((size_t)g.nv + g.nt + g.lr));
     // S_z is hermitian, so the particle (isign = +1) and hole (-1) terms come
     // from one chain (build_chi_spin.f90:186-250)
     std::vector<ChiTerm> terms;
     for (int isign = 1; isign >= -1; isign -= 2)
         terms.push_back(ChiTerm{alpha, beta_l, nlanc, 0, isign, 1, peso_f, 0.0, peso_bz, ei});
+    if (chi_route(terms, g) < 0) {
+        std::vector<double> d(alpha, alpha + nlanc), e(nlanc, 0.0), z(nlanc);
+        for (int i = 1; i < nlanc; ++i) e[i] = beta_l[i];
+        if (tql2_first_row(nlanc, d.data(), e.data(), z.data()))
+            return fail(DMED_ENOCONV, "tql2 did not converge");
+        for (auto &x : z) x = x * x;
+        for (const ChiTerm &t : terms)
+            chi_add_branch(peso_f, 0.0, peso_bz, ei, d.data(), z.data(), nlanc, t.isign, 1, beta, vm,
+                           g.nv, tau, g.nt, wr, g.lr, eps, chi_iv, chi_tau, chi_w);
+        return 0;
+    }
+    std::vector<double> o(2 * ((size_t)g.nv + g.nt + g.lr));
     if (int rc = chi_sum(terms, 1, beta, g, o.data())) return rc;
     for (int i = 0; i < 2 * g.nv; ++i) chi_iv[i] += o[i];
     for (int i = 0; i < g.nt; ++i) chi_tau[i] += o[2 * ((size_t)g.nv + i)];

@@ -387,6 +387,8 @@ struct GfTerm {
     int n, isign;
     double ei, pr, pi;
 };
+bool gf_on_device(const std::vector<GfTerm> &terms, const double *wm, int lm, const double *wr, int lr,
+                  double eps);
 // sum of the terms on both axes (gf.hip): g[0..lm) at i*wm, g[lm..lm+lr) at
 // wr + i*eps, interleaved complex, overwritten
 int gf_sum(const std::vector<GfTerm> &terms, const double *wm, int lm, const double *wr, int lr,
@@ -404,6 +406,7 @@ struct ChiGrid {
     int nv, nt, lr;
     double eps;
 };
+int chi_route(const std::vector<ChiTerm> &terms, const ChiGrid &g);     // -1: on the host
 // sums of the terms (gf.hip): out[target*(nv+nt+lr) + i], interleaved complex
 // (tau: real part), overwritten
 int chi_sum(std::vector<ChiTerm> terms, int ntarget, double beta, const ChiGrid &g, double *out);

@@ -20,10 +20,12 @@
 // at Ns = 8 (200 steps), 25.3 -> 19.0 ms at Ns = 12 (300 steps); error of
 // G(iw) against 64-bit pole sums 1e-14 and 5e-14, both ways alike.
 #include <algorithm>
+#include <atomic>
 #include <cfloat>
 #include <cmath>
 #include <complex>
 #include <cstring>
+#include <thread>
 #include <vector>
 
 #include "dmed_internal.h"
@@ -169,15 +171,16 @@ int gf_sum_host(const std::vector<GfTerm> &terms, const double *wm, int lm, cons
 // ------------------------------------------------------- susceptibilities
 // The susceptibility sums (build_chi_spin.f90:186-250, build_chi_dens.f90:
 // 505-733) weigh every pole with exp(-beta dE) and need chi(tau), so they
-// take the poles themselves.  k_chain_poles finds them (the implicit QL
-// iteration of tql2_first_row, one wave per chain, all chains of a solve in
-// one launch), k_chi_prep turns them into the factors that do not depend on
+// take the poles themselves.  k_chain_poles finds those of many chains (the
+// implicit QL iteration of tql2_first_row, one wave per chain, all chains of a
+// solve in one launch), the host those of a few; k_chi_prep turns them into the factors that do not depend on
 // the frequency, k_chi_term sums one term's poles at one point per thread
 // and k_chi_sum adds a target's terms in order.
 //
 // The QL recurrence is serial (about 0.8 n^2 rotations, each one reciprocal
-// square root after the other), so a chain costs its latency; on the host
-// it took 2.3 ms per 200-step chain and the sums another 3.2 ms per chain.
+// square root after the other), so a chain costs its latency, 190 n^2 ns here
+// and 37 n^2 ns on the host (200 steps: 7.7 and 1.5 ms): the launch pays from
+// about 40 chains on eight host threads, or five on one (chi_route).
 // Measured on a two-orbital Ns = 8 solve at beta = 100 with both
 // susceptibilities (40 to 200 chains): 374 -> 213 ms.
 
@@ -321,9 +324,44 @@ __global__ void __launch_bounds__(64) k_chi_sum(const ChiDev *__restrict__ t, in
 // terms of one launch: bounds the partial results to kChiBatch*np*16 bytes
 constexpr int kChiBatch = 256;
 
-// terms sorted by target
+// poles of the chains on nthread host threads, the longest first: over the
+// coefficient pairs, as k_chain_poles would leave them
+int chi_poles_host(const std::vector<PoleChain> &ch, int nthread, double *ab)
+{
+    std::vector<int> order(ch.size());
+    for (size_t k = 0; k < ch.size(); ++k) order[k] = (int)k;
+    std::stable_sort(order.begin(), order.end(), [&](int x, int y) { return ch[x].n > ch[y].n; });
+    std::atomic<size_t> next(0);
+    std::atomic<int> bad(0);
+    auto work = [&]() {
+        std::vector<double> d, e, z;
+        for (size_t k; (k = next.fetch_add(1)) < order.size();) {
+            const PoleChain c = ch[order[k]];
+            double *p = ab + 2 * (size_t)c.off;
+            d.resize(c.n);
+            e.resize(c.n);
+            z.resize(c.n);
+            for (int i = 0; i < c.n; ++i) {
+                d[i] = p[2 * i];
+                e[i] = p[2 * i + 1];
+            }
+            if (tql2_first_row(c.n, d.data(), e.data(), z.data())) bad = 1;
+            for (int i = 0; i < c.n; ++i) {
+                p[2 * i] = d[i];
+                p[2 * i + 1] = z[i] * z[i];
+            }
+        }
+    };
+    std::vector<std::thread> th;
+    for (int t = 1; t < nthread; ++t) th.emplace_back(work);
+    work();
+    for (auto &t : th) t.join();
+    return bad ? fail(DMED_ENOCONV, "tql2 did not converge") : 0;
+}
+
+// terms sorted by target; nthread > 0: poles on that many host threads
 int chi_sum_device(const std::vector<ChiTerm> &terms, int ntarget, double beta, const ChiGrid &g,
-                   double *out)
+                   double *out, int nthread)
 {
     hipStream_t st = ex().stream;
     const int np = g.nv + g.nt + g.lr, nterm = (int)terms.size();
@@ -350,6 +388,8 @@ int chi_sum_device(const std::vector<ChiTerm> &terms, int ntarget, double beta, 
         ++toff[t.target + 1];
     }
     for (int q = 0; q < ntarget; ++q) toff[q + 1] += toff[q];
+    if (nthread > 0)
+        if (int rc = chi_poles_host(ch, nthread, ab.data())) return rc;
     const size_t nch = ch.size();
     auto up = [](size_t b) { return (b + 255) & ~(size_t)255; };
     const size_t ox = 0, och = ox + up((size_t)np * 8), odev = och + up(nch * sizeof(PoleChain));
@@ -371,14 +411,15 @@ int chi_sum_device(const std::vector<ChiTerm> &terms, int ntarget, double beta, 
     if (int rc = exec_try(ex(), kSlotGf, total, (void **)&d)) return rc;
     DMED_HIP(hipMemcpyAsync(d, h.data(), nup, hipMemcpyHostToDevice, st));
     const ChiDev *dt = reinterpret_cast<const ChiDev *>(d + odev);
-    double2 *dpole = reinterpret_cast<double2 *>(d + opole);
+    double2 *dpole = reinterpret_cast<double2 *>(d + (nthread > 0 ? oab : opole));
     double4 *dfac = reinterpret_cast<double4 *>(d + ofac);
     double2 *dout = reinterpret_cast<double2 *>(d + oout);
     double2 *dpart = reinterpret_cast<double2 *>(d + opart);
-    hipLaunchKernelGGL(k_chain_poles, dim3((unsigned)nch), dim3(64), (size_t)nmax * 24, st,
-                       reinterpret_cast<const PoleChain *>(d + och),
-                       reinterpret_cast<const double2 *>(d + oab), dpole,
-                       reinterpret_cast<int32_t *>(d + ost));
+    if (nthread == 0)
+        hipLaunchKernelGGL(k_chain_poles, dim3((unsigned)nch), dim3(64), (size_t)nmax * 24, st,
+                           reinterpret_cast<const PoleChain *>(d + och),
+                           reinterpret_cast<const double2 *>(d + oab), dpole,
+                           reinterpret_cast<int32_t *>(d + ost));
     const unsigned gx = (unsigned)((np + 63) / 64);
     for (int c0 = 0; c0 < nterm; c0 += kChiBatch) {
         const int nc = std::min(kChiBatch, nterm - c0);
@@ -391,8 +432,9 @@ int chi_sum_device(const std::vector<ChiTerm> &terms, int ntarget, double beta, 
                            reinterpret_cast<const int32_t *>(d + otoff), dpart, g.nv, g.nt, np, dout);
     }
     DMED_HIP(hipGetLastError());
-    std::vector<int32_t> bad(nch);
-    DMED_HIP(hipMemcpyAsync(bad.data(), d + ost, nch * 4, hipMemcpyDeviceToHost, st));
+    std::vector<int32_t> bad(nch, 0);
+    if (nthread == 0)
+        DMED_HIP(hipMemcpyAsync(bad.data(), d + ost, nch * 4, hipMemcpyDeviceToHost, st));
     DMED_HIP(hipMemcpyAsync(out, dout, (size_t)ntarget * np * 16, hipMemcpyDeviceToHost, st));
     DMED_HIP(hipStreamSynchronize(st));
     for (int32_t b : bad)
@@ -433,57 +475,90 @@ int chi_sum_host(const std::vector<ChiTerm> &terms, double beta, const ChiGrid &
 // goes to the caller.
 bool host_may_take(int rc) { return rc == DMED_ENOMEM || rc == DMED_ENOCONV; }
 
-// g[0..lm) on the Matsubara axis, g[lm..lm+lr) on the real axis, overwritten
-// with the sum over the terms.  The continued fraction needs every point off
-// the real axis (1e-100: its square is still a normal number) and finite
-// coefficients.  Chains under kCfMin steps stay on the host: their poles cost
-// it 10-20 us there, less than the upload, the two launches and the download.
-int gf_sum(const std::vector<GfTerm> &terms, const double *wm, int lm, const double *wr, int lr,
-           double eps, double *g)
+// Whether a sum runs on the device.  The continued fraction needs every point
+// off the real axis (1e-100: its square is still a normal number) and finite
+// coefficients.  The upload, two launches and the download take 36 us; the
+// host takes 50 n^2 ns for the poles of a short chain and 0.5 ns per pole and
+// frequency (n = 20: 22 us at 8 frequencies, 27 at 512; n = 10 at 4596: 33).
+bool gf_on_device(const std::vector<GfTerm> &terms, const double *wm, int lm, const double *wr, int lr,
+                  double eps)
 {
-    constexpr int kCfMin = 16;
-    int nmax = 0;
+    constexpr double kDeviceNs = 36e3;
+    double host_ns = 0.0;
     bool ok = ctx().initialized && lm + lr > 0;
     for (const GfTerm &t : terms) {
-        nmax = std::max(nmax, t.n);
+        host_ns += (50.0 * t.n + 0.5 * ((double)lm + lr)) * t.n;
         for (int i = 0; i < t.n && ok; ++i)
             ok = std::fabs(t.alpha[i]) < 1e100 && (i == 0 || std::fabs(t.beta[i]) < 1e100);
         ok = ok && std::fabs(t.ei) < 1e100 && (t.isign == 1 || t.isign == -1);
     }
-    ok = ok && nmax >= kCfMin && (lr == 0 || (std::fabs(eps) > 1e-100 && std::fabs(eps) < 1e100));
+    ok = ok && host_ns > kDeviceNs && (lr == 0 || (std::fabs(eps) > 1e-100 && std::fabs(eps) < 1e100));
     for (int i = 0; i < lm && ok; ++i) ok = std::fabs(wm[i]) > 1e-100 && std::fabs(wm[i]) < 1e100;
     for (int i = 0; i < lr && ok; ++i) ok = std::fabs(wr[i]) < 1e100;
-    if (ok) {
+    return ok;
+}
+
+// g[0..lm) on the Matsubara axis, g[lm..lm+lr) on the real axis, overwritten
+// with the sum over the terms
+int gf_sum(const std::vector<GfTerm> &terms, const double *wm, int lm, const double *wr, int lr,
+           double eps, double *g)
+{
+    if (gf_on_device(terms, wm, lm, wr, lr, eps)) {
         const int rc = gf_sum_device(terms, wm, lm, wr, lr, eps, g);
         if (!host_may_take(rc)) return rc;
     }
     return gf_sum_host(terms, wm, lm, wr, lr, eps, g);
 }
 
+// Where a susceptibility sum runs, terms sorted by target: -1 on the host; else
+// on the device, with the poles on that many host threads, 0: on the device
+// too.  Coefficients that are not finite go to the host.  Measured: a wave
+// takes 60 us and 190 n^2 ns for the poles of a chain, the host 37 n^2 ns;
+// the sums cost the device 45 us and 0.4 us per pole of the longest chain, and
+// the host 0.8 ns per pole of a term and point of the iv and real axes and 2.8
+// ns per point of the tau axis.  One chain of 200 steps, 1626 points: 2.05 ms
+// on the host alone, 1.55 ms with the sums here, 7.8 ms with the poles here too.
+// Threads of a solve's own (sites) take their chains alone.
+int chi_route(const std::vector<ChiTerm> &terms, const ChiGrid &g)
+{
+    constexpr int kMaxSteps = 2048;             // 3 doubles a step in LDS
+    constexpr int kThreads = 8;
+    double nmax = 0.0, sq = 0.0, sum_ns = 0.0;
+    size_t nsum = 0, nch = 0;
+    const double *last = nullptr;
+    bool ok = ctx().initialized && g.nv + g.nt + g.lr > 0;
+    for (const ChiTerm &t : terms) {
+        nsum += t.n;
+        sum_ns += t.n * (0.8 * ((double)g.nv + g.lr) + 2.8 * g.nt);
+        if (t.alpha != last) {
+            nmax = std::max(nmax, (double)t.n);
+            sq += (double)t.n * t.n;
+            ++nch;
+        }
+        last = t.alpha;
+        for (int i = 0; i < t.n && ok; ++i)
+            ok = std::fabs(t.alpha[i]) < 1e100 && (i == 0 || std::fabs(t.beta[i]) < 1e100);
+    }
+    if (!ok || nsum >= ((size_t)1 << 24)) return -1;        // 64 B of work space a pole
+    // threads where the chains take longer than starting them
+    const int nthread = &ex() == &ctx().exec && 37.0 * sq > 300e3 ? (int)std::min<size_t>(nch, kThreads) : 1;
+    const double host_ns = 37.0 * std::max(nmax * nmax, sq / nthread);
+    if (nmax <= kMaxSteps && host_ns > 60e3 + 190.0 * nmax * nmax) return 0;
+    return sum_ns > 45e3 + 400.0 * nmax ? nthread : -1;
+}
+
 // out[target * np + i], np = nv + nt + lr points (iv, tau, real axis),
 // interleaved complex (tau: its real part), overwritten with the sums over
-// the terms.  Chains under kChiMin steps take the host less than the launches;
-// coefficients that are not finite go there too, for tql2's error.
+// the terms
 int chi_sum(std::vector<ChiTerm> terms, int ntarget, double beta, const ChiGrid &g, double *out)
 {
-    constexpr int kChiMin = 16;
-    constexpr int kChiMaxSteps = 2048;          // 3 doubles a step in LDS
     std::fill(out, out + 2 * (size_t)ntarget * (g.nv + g.nt + g.lr), 0.0);
     if (terms.empty()) return 0;
     std::stable_sort(terms.begin(), terms.end(),
                      [](const ChiTerm &a, const ChiTerm &b) { return a.target < b.target; });
-    int nmax = 0;
-    size_t nsum = 0;
-    bool ok = ctx().initialized && g.nv + g.nt + g.lr > 0;
-    for (const ChiTerm &t : terms) {
-        nmax = std::max(nmax, t.n);
-        nsum += t.n;
-        for (int i = 0; i < t.n && ok; ++i)
-            ok = std::fabs(t.alpha[i]) < 1e100 && (i == 0 || std::fabs(t.beta[i]) < 1e100);
-    }
-    ok = ok && nmax >= kChiMin && nmax <= kChiMaxSteps && nsum < ((size_t)1 << 24);     // 64 B of work space a pole
-    if (ok) {
-        const int rc = chi_sum_device(terms, ntarget, beta, g, out);
+    const int route = chi_route(terms, g);
+    if (route >= 0) {
+        const int rc = chi_sum_device(terms, ntarget, beta, g, out, route);
         if (!host_may_take(rc)) return rc;
     }
     std::fill(out, out + 2 * (size_t)ntarget * (g.nv + g.nt + g.lr), 0.0);
