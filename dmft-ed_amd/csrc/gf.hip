@@ -25,6 +25,7 @@
 #include <cmath>
 #include <complex>
 #include <cstring>
+#include <system_error>
 #include <thread>
 #include <vector>
 
@@ -353,7 +354,11 @@ int chi_poles_host(const std::vector<PoleChain> &ch, int nthread, double *ab)
         }
     };
     std::vector<std::thread> th;
-    for (int t = 1; t < nthread; ++t) th.emplace_back(work);
+    try {
+        for (int t = 1; t < nthread; ++t) th.emplace_back(work);
+    } catch (const std::system_error &) {
+        // fewer threads than asked for
+    }
     work();
     for (auto &t : th) t.join();
     return bad ? fail(DMED_ENOCONV, "tql2 did not converge") : 0;
