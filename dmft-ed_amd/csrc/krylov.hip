@@ -996,12 +996,13 @@ int chain_init(const dmed_sector *s, void *bufs[3], int prec, int nlanc_total, d
 }
 
 // Lanczos steps are captured into a HIP graph when a run is long enough:
-// three steps bring the (v_prev, v, w) rotation back to the start, so one
-// captured three-step graph is replayed.  DMED_GRAPHS=0 turns this off.
+// three steps bring the (v_prev, v, w) rotation back to the start, six also the
+// two sets of scalars of the two-launch step, so one captured graph of that
+// many steps is replayed.  DMED_GRAPHS=0 turns this off.
 constexpr int kGraphMinSteps = 30;
 
-// DMED_TEST_CAPTURE_FAIL=q makes step q (0..2) of the captured three-step
-// window fail before it is recorded: a test of the fallback to eager steps.
+// DMED_TEST_CAPTURE_FAIL=q makes step q of the captured window (0..2 or 0..5)
+// fail before it is recorded: a test of the fallback to eager steps.
 static int capture_fail_step()
 {
     static const int q = [] {
