@@ -19,7 +19,7 @@
 // The algorithm is the one of trl_run / trl_deflated (krylov.hip): the same
 // start vectors, three-term steps, restart rule, convergence test and
 // keep/evict rules.  A pair of steps whose norm comes out too small falls back
-// to passes of its own here at once (on the host the cycle is taken again), and
+// to passes of its own here at once (on the host the rest of the cycle is taken again), and
 // the eigensolver of the projected matrix differs (Jacobi here, Householder + QL
 // on the host), so results agree to the solver tolerance rather than bit for
 // bit.
