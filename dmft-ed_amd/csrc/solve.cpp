@@ -532,6 +532,9 @@ extern "C" int dmed_solve(const dmed_solve_params *p, dmed_solve_out *out)
             r.ev = it.evals;
             r.vecs = std::move(it.vecs);
             it.vecs.clear();
+            if (p->verbose > 1)
+                std::fprintf(stderr, "sector %d dim=%lld neig=%d nout=%d dense batch\n", dsec[k],
+                             (long long)it.s->dim, it.neig, it.nout);
         }
         const int frc = queue_finish(q);
         if (!qrc) qrc = frc;
