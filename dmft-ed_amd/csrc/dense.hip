@@ -12,9 +12,10 @@
 // beside four Krylov sectors): 101 -> 30 ms.
 //
 // Bounds: the reduction streams the trailing matrix from L2 three times a
-// step (2.9 ms of the 12 ms at 225 states, eight columns in flight); the QL recurrence is serial, so wave 0 runs it one sweep ahead of the
-// other waves, which apply the rotations of the sweep before to the rows of
-// Z (a lane per row, coalesced along the column).  Z and H stay in the
+// step (2.9 ms of the 12 ms at 225 states, eight columns in flight); the QL
+// recurrence is serial, so wave 0 runs it one sweep ahead of the other waves,
+// which apply the rotations of the sweep before to the rows of Z (a lane per
+// row, coalesced along the column).  Z and H stay in the
 // XCD's L2 (2 x 405 KB at 225 states).
 #include <algorithm>
 #include <cmath>

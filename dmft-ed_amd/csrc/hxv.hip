@@ -221,7 +221,7 @@ __global__ void __launch_bounds__(1024) k_hxv(const HxvArgs<T> a)
 // upper byte indexes a table of signed coefficients: four VALU operations a
 // hop besides the product, where unpacking and 64-bit addresses took eleven
 // (FP32, D = 1.2e7, two orbitals: 106 -> 81 us; FP64, D = 2.2e6: 26 -> 22 us;
-// the largest sector: FP64 1.98 -> 1.85 ms, FP32 1.06 -> 0.98 ms, back to back).
+// the largest sector: FP64 2.01 -> 1.97 ms, FP32 1.07 -> 0.98 ms).
 // HALVES = 2: steps 2-4 run twice, for the first and the second half of the
 // lane's rows, one neighbour column at a time.  Half the accumulators, loads
 // and hop words are live at once, which brings the kernel within the
