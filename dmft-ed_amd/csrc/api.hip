@@ -698,7 +698,7 @@ extern "C" int dmed_gf_add_chain(double peso_bz, double ei, const double *alpha,
         return 0;
     }
     std::vector<double> g(2 * ((size_t)lm + lr));
-    if (int rc = gf_sum(term, wm, lm, wr, lr, eps, g.data())) return rc;
+    if (int rc = gf_sum(term, wm, lm, wr, lr, eps, g.data(), true)) return rc;
     for (size_t i = 0; i < 2 * (size_t)lm; ++i) gmats[i] += g[i];
     for (size_t i = 0; i < 2 * (size_t)lr; ++i) greal[i] += g[2 * (size_t)lm + i];
     return 0;
@@ -935,7 +935,8 @@ extern "C" int dmed_chi_add_chain(double peso_f, double peso_bz, double ei, cons
     std::vector<ChiTerm> terms;
     for (int isign = 1; isign >= -1; isign -= 2)
         terms.push_back(ChiTerm{alpha, beta_l, nlanc, 0, isign, 1, peso_f, 0.0, peso_bz, ei});
-    if (chi_route(terms, g) < 0) {
+    const int route = chi_route(terms, g);
+    if (route < 0) {
         std::vector<double> d(alpha, alpha + nlanc), e(nlanc, 0.0), z(nlanc);
         for (int i = 1; i < nlanc; ++i) e[i] = beta_l[i];
         if (tql2_first_row(nlanc, d.data(), e.data(), z.data()))
@@ -947,7 +948,7 @@ extern "C" int dmed_chi_add_chain(double peso_f, double peso_bz, double ei, cons
         return 0;
     }
     std::vector<double> o(2 * ((size_t)g.nv + g.nt + g.lr));
-    if (int rc = chi_sum(terms, 1, beta, g, o.data())) return rc;
+    if (int rc = chi_sum(terms, 1, beta, g, o.data(), &route)) return rc;
     for (int i = 0; i < 2 * g.nv; ++i) chi_iv[i] += o[i];
     for (int i = 0; i < g.nt; ++i) chi_tau[i] += o[2 * ((size_t)g.nv + i)];
     for (int i = 0; i < 2 * g.lr; ++i) chi_w[i] += o[2 * ((size_t)g.nv + g.nt) + i];

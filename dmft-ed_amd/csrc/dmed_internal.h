@@ -390,9 +390,10 @@ struct GfTerm {
 bool gf_on_device(const std::vector<GfTerm> &terms, const double *wm, int lm, const double *wr, int lr,
                   double eps);
 // sum of the terms on both axes (gf.hip): g[0..lm) at i*wm, g[lm..lm+lr) at
-// wr + i*eps, interleaved complex, overwritten
+// wr + i*eps, interleaved complex, overwritten; on_device: gf_on_device of the
+// same arguments
 int gf_sum(const std::vector<GfTerm> &terms, const double *wm, int lm, const double *wr, int lr,
-           double eps, double *g);
+           double eps, double *g, bool on_device);
 // One branch of a susceptibility: the poles of (alpha[0..n), beta[1..n)) with
 // weight (pr + i pi)*peso_bz added to output `target`.
 struct ChiTerm {
@@ -409,7 +410,8 @@ struct ChiGrid {
 int chi_route(const std::vector<ChiTerm> &terms, const ChiGrid &g);     // -1: on the host
 // sums of the terms (gf.hip): out[target*(nv+nt+lr) + i], interleaved complex
 // (tau: real part), overwritten
-int chi_sum(std::vector<ChiTerm> terms, int ntarget, double beta, const ChiGrid &g, double *out);
+int chi_sum(std::vector<ChiTerm> terms, int ntarget, double beta, const ChiGrid &g, double *out,
+            const int *known_route = nullptr);
 // one branch of the susceptibility pole sums (build_chi_spin.f90:186-250,
 // build_chi_dens.f90:505-733): complex weight pr + i pi, iv = 0 term signed
 // by iv0_sign; vm[0..nv), tau[0..ntau), wr[0..lreal); chi_iv, chi_w

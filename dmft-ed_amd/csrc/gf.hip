@@ -506,9 +506,9 @@ bool gf_on_device(const std::vector<GfTerm> &terms, const double *wm, int lm, co
 // g[0..lm) on the Matsubara axis, g[lm..lm+lr) on the real axis, overwritten
 // with the sum over the terms
 int gf_sum(const std::vector<GfTerm> &terms, const double *wm, int lm, const double *wr, int lr,
-           double eps, double *g)
+           double eps, double *g, bool on_device)
 {
-    if (gf_on_device(terms, wm, lm, wr, lr, eps)) {
+    if (on_device) {
         const int rc = gf_sum_device(terms, wm, lm, wr, lr, eps, g);
         if (!host_may_take(rc)) return rc;
     }
@@ -527,7 +527,7 @@ int gf_sum(const std::vector<GfTerm> &terms, const double *wm, int lm, const dou
 int chi_route(const std::vector<ChiTerm> &terms, const ChiGrid &g)
 {
     constexpr int kMaxSteps = 2048;             // 3 doubles a step in LDS
-    constexpr int kThreads = 8;
+    static const size_t kThreads = std::min(8u, std::max(1u, std::thread::hardware_concurrency()));
     double nmax = 0.0, sq = 0.0, sum_ns = 0.0;
     size_t nsum = 0, nch = 0;
     const double *last = nullptr;
@@ -546,7 +546,7 @@ int chi_route(const std::vector<ChiTerm> &terms, const ChiGrid &g)
     }
     if (!ok || nsum >= ((size_t)1 << 24)) return -1;        // 64 B of work space a pole
     // threads where the chains take longer than starting them
-    const int nthread = &ex() == &ctx().exec && 37.0 * sq > 300e3 ? (int)std::min<size_t>(nch, kThreads) : 1;
+    const int nthread = &ex() == &ctx().exec && 37.0 * sq > 300e3 ? (int)std::min(nch, kThreads) : 1;
     const double host_ns = 37.0 * std::max(nmax * nmax, sq / nthread);
     if (nmax <= kMaxSteps && host_ns > 60e3 + 190.0 * nmax * nmax) return 0;
     return sum_ns > 45e3 + 400.0 * nmax ? nthread : -1;
@@ -555,13 +555,14 @@ int chi_route(const std::vector<ChiTerm> &terms, const ChiGrid &g)
 // out[target * np + i], np = nv + nt + lr points (iv, tau, real axis),
 // interleaved complex (tau: its real part), overwritten with the sums over
 // the terms
-int chi_sum(std::vector<ChiTerm> terms, int ntarget, double beta, const ChiGrid &g, double *out)
+int chi_sum(std::vector<ChiTerm> terms, int ntarget, double beta, const ChiGrid &g, double *out,
+            const int *known_route)
 {
     std::fill(out, out + 2 * (size_t)ntarget * (g.nv + g.nt + g.lr), 0.0);
     if (terms.empty()) return 0;
     std::stable_sort(terms.begin(), terms.end(),
                      [](const ChiTerm &a, const ChiTerm &b) { return a.target < b.target; });
-    const int route = chi_route(terms, g);
+    const int route = known_route ? *known_route : chi_route(terms, g);
     if (route >= 0) {
         const int rc = chi_sum_device(terms, ntarget, beta, g, out, route);
         if (!host_may_take(rc)) return rc;

@@ -835,7 +835,8 @@ extern "C" int dmed_solve(const dmed_solve_params *p, dmed_solve_out *out)
                 if (ch.kind != 0 || ch.s != s || ch.a != a || !(ch.norm2 > 0.0)) continue;
                 terms.push_back(term_of(ch));
             }
-            if ((rc = gf_sum(terms, wm.data(), lm, wr.data(), lr, p->eps, gsum.data()))) break;
+            if ((rc = gf_sum(terms, wm.data(), lm, wr.data(), lr, p->eps, gsum.data(),
+                             gf_on_device(terms, wm.data(), lm, wr.data(), lr, p->eps)))) break;
             std::copy(gsum.begin(), gsum.begin() + 2 * (size_t)lm, gm.begin());
             std::copy(gsum.begin() + 2 * (size_t)lm, gsum.end(), gr.begin());
             for (int l = 0; l < lm && out->gmats; ++l) {
@@ -891,7 +892,8 @@ extern "C" int dmed_solve(const dmed_solve_params *p, dmed_solve_out *out)
                         continue;
                     terms.push_back(term_of(ch));
                 }
-                if ((rc = gf_sum(terms, wm.data(), lm, wr.data(), lr, p->eps, gsum.data()))) break;
+                if ((rc = gf_sum(terms, wm.data(), lm, wr.data(), lr, p->eps, gsum.data(),
+                             gf_on_device(terms, wm.data(), lm, wr.data(), lr, p->eps)))) break;
                 std::vector<double> am(gsum.begin(), gsum.begin() + 2 * (size_t)lm),
                     ar(gsum.begin() + 2 * (size_t)lm, gsum.end());
                 auto combine = [&](std::vector<double> &g, const std::vector<double> &full, int L) {
